@@ -151,6 +151,27 @@ def test_gemm_rows_bits(xm, xo, n_tok, n_out, n_in):
     assert np.array_equal(got.view(np.uint32), xo.gemm_rows(x, w).view(np.uint32))
 
 
+@pytest.mark.parametrize("n_tok,n_out,n_in,ld", [
+    (9, 63, 127, 127), (64, 64, 128, 128), (65, 64, 130, 133), (17, 65, 144, 144), (16, 200, 1, 1), (1, 1, 272, 272),
+    (130, 3, 400, 401), (33, 128, 640, 642), (1100, 130, 400, 401), (9000, 5, 144, 144), (1030, 255, 129, 131)])
+def test_gemm_rows_edges(xm, xo, n_tok, n_out, n_in, ld):
+    """The chains' bits at the edges of both forms' tiles (16 x 16 rows up to 512 work-groups, else 64 x 16; steps of 256
+    and 128 values, 16 at a time): odd sizes, weights or tokens over the lanes, x rows at any float's address, and values
+    whose products and sums leave the normal range."""
+    rng = np.random.default_rng(n_tok * n_in + n_out)
+    x = rng.standard_normal((n_tok, n_in)).astype(np.float32)
+    w = rng.standard_normal((n_out, n_in)).astype(np.float32)
+    x[1::4] *= np.float32(1e-20)                        # subnormal products with the scaled weight rows
+    w[::3] *= np.float32(1e-22)
+    x[::5, ::7] = 0.0
+    x[2::6] = -0.0
+    buf = torch.zeros(n_tok * (ld + 1) + 1, device=DEV)   # rows ld + 1 floats apart, from the second float on
+    xd = buf[1:].view(n_tok, ld + 1)[:, :n_in]
+    xd.copy_(torch.from_numpy(x))
+    got = t2n(xm.f32_gemm_rows(xd, torch.from_numpy(w).to(DEV)))
+    assert np.array_equal(got.view(np.uint32), xo.gemm_rows(x, w).view(np.uint32))
+
+
 def test_f32_to_bf16_reference_vectors(xm, golden):
     """f32_to_bf16_bulk against the reference's own bf16_from_f32 outputs (committed vectors: ties, carries,
     overflow to inf, NaNs kept quiet)."""

@@ -22,6 +22,8 @@
 #include "xs_device.h"
 #include "xs_kernels.h"
 
+#include <type_traits>
+
 namespace xs {
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return u2f((uint32_t)b << 16); }
@@ -116,65 +118,169 @@ template hipError_t launch_mmvf<float>(const float*, int64_t, const float*, floa
 template hipError_t launch_mmvf<uint16_t>(const float*, int64_t, const uint16_t*, float*, int64_t, int64_t, int64_t,
                                           int, hipStream_t);
 
-// 64 tokens x 64 rows a work-group; thread (ti, tj) = (tid / 16, tid % 16) owns tokens 4 ti .. and rows 4 tj ..
-constexpr int kGT = 64, kGK = 32;
-__global__ __launch_bounds__(256) void gemm_rows_kernel(const float* __restrict__ x, int64_t ldx,
-                                                        const float* __restrict__ w, float* __restrict__ y,
-                                                        int64_t ldy, int64_t n_in, int64_t n_out, int64_t n_tok) {
-    __shared__ float4 xs[kGK][kGT / 4];
-    __shared__ float4 ws[kGK][kGT / 4];
-    const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
-    const int64_t t0 = (int64_t)blockIdx.y * kGT, o0 = (int64_t)blockIdx.x * kGT;
-    const int64_t k_end = (n_in + 15) / 16 * 16;   // the reference's chain: zeros up to a multiple of 16
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-    // loader: thread tid reads 8 consecutive k of token / row (tid / 4) at k offset 8 (tid % 4)
-    const int lr = tid >> 2, lk = (tid & 3) * 8;
-    for (int64_t k0 = 0; k0 < k_end; k0 += kGK) {
-        float xv[8], wv[8];
-        const int64_t tr = t0 + lr, wr = o0 + lr;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t k = k0 + lk + u;
-            xv[u] = tr < n_tok && k < n_in ? x[tr * ldx + k] : 0.0f;
-            wv[u] = wr < n_out && k < n_in ? w[wr * n_in + k] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            ((float*)&xs[lk + u][0])[lr] = xv[u];
-            ((float*)&ws[lk + u][0])[lr] = wv[u];
-        }
-        __syncthreads();
-        const int kn = (int)min((int64_t)kGK, k_end - k0);
-        for (int kk = 0; kk < kn; ++kk) {
-            const float4 a = xs[kk][ti], b = ws[kk][tj];
-            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(av[i], bv[j], acc[i][j]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t t = t0 + 4 * ti + i;
-        if (t >= n_tok) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t o = o0 + 4 * tj + j;
-            if (o < n_out) y[t * ldy + o] = acc[i][j];
-        }
+// The gemm_rows chains.  One side's rows (weights or tokens) lie over the lanes, their values staged through LDS; the
+// other side's ("group rows") stay one value a lane in registers and are broadcast by the multiply-add itself, so the
+// inner loop has no other instruction than its multiply-adds and the lane rows' LDS reads.  Two forms:
+//   few chains: 16 lane rows x 4 group rows a wave, v_fmac_f32 whose DPP operand takes lane kk of each 16
+//     (row_newbcast; lane i of the 16: the group row's value at k0 + i).  A work-group reads 32 rows: with few
+//     work-groups one compute unit's share of the memory system bounds it, not the chip's (64-row tiles: 2048 x 1 x 64
+//     tokens 20.3 us against 14.6).
+//   many chains: v_mfma_f32_4x4x1_16b_f32, one FMA (one rounding) an output: a run of them over k = 0, 1, ... is the
+//     chain itself.  64 lane rows x 4 group rows a wave; lane 4 kk + i holds group row i at k0 + kk, and CBSZ 4 / ABID
+//     kk broadcast block kk.  A row is then read by fewer work-groups (8 group rows a wave in two accumulators, two
+//     waves a work-group: 2048 tokens 34.6 us against 26.3).
+// Chains are 1024 to 7168 steps long and few (2048 tokens x 128 experts: 4 a lane of the whole chip), so their length
+// is what bounds a router: about 14 cycles a step as measured.  The loads ahead must not stop it: two steps ahead through
+// registers, then LDS.  A tile of 64 x 64 chains a work-group, 4 x 4 a thread, read from LDS a k at a time and waiting
+// for each step's loads, took 230 us at 2048 tokens x 128 experts x 2048 (now 25; 62 against 17 TFLOP/s at 4096 x 256 x
+// 7168), and 165 us for one weight row x 64 tokens x 2048 (now 13).
+struct __attribute__((packed, aligned(4))) F4u {   // 16 bytes at any float's address
+    float v[4];
+};
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// 16 steps of a wave's chains, few-chains form: acc = fma(group value kk of the lane's 16, b[kk], acc), kk = 0 .. 15.
+// (One block: the compiler makes a move of every broadcast.  The s_nop covers a group value written by the instruction
+// before, which a DPP read has to stay two wait states behind.)
+#define XS_FMAC(KK, B) "v_fmac_f32_dpp %0, %1, " B " row_newbcast:" KK " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void chain16(float& acc, float g, const float (&b)[16]) {
+    asm("s_nop 1\n\t" XS_FMAC("0", "%2") XS_FMAC("1", "%3") XS_FMAC("2", "%4") XS_FMAC("3", "%5") XS_FMAC("4", "%6")
+            XS_FMAC("5", "%7") XS_FMAC("6", "%8") XS_FMAC("7", "%9") XS_FMAC("8", "%10") XS_FMAC("9", "%11")
+                XS_FMAC("10", "%12") XS_FMAC("11", "%13") XS_FMAC("12", "%14") XS_FMAC("13", "%15") XS_FMAC("14", "%16")
+                    XS_FMAC("15", "%17")
+        : "+v"(acc)
+        : "v"(g), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]),
+          "v"(b[9]), "v"(b[10]), "v"(b[11]), "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
+}
+#undef XS_FMAC
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+template <int KK>
+__device__ __forceinline__ void mfma16(f32x4_t& acc, float g, const float (&b)[16]) {
+    if constexpr (KK < 16) {
+        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(g, b[KK], acc, 4, KK, 0);
+        mfma16<KK + 1>(acc, g, b);
     }
 }
 
+// y[p * yl + q * yg] = lane row p . group row q.  A work-group: LR lane rows x 16 group rows, 4 waves, KS values a
+// step.  In LDS 16-byte chunk c of row r lies at c ^ (r % 16): the reads of 16 lanes cover all banks once.
+template <bool MANY>
+__global__ __launch_bounds__(256) void gemm_rows_kernel(const float* __restrict__ lanes, int64_t ldl,
+                                                                     int64_t n_l, const float* __restrict__ groups,
+                                                                     int64_t ldg, int64_t n_g, float* __restrict__ y,
+                                                                     int64_t yl, int64_t yg, int64_t n_in,
+                                                                     unsigned lane_tiles) {
+    constexpr int LR = MANY ? 64 : 16, KS = MANY ? 128 : 256;
+    constexpr int kChunks = KS / 4, kLd = LR * kChunks / 256, kRowStep = 256 / kChunks;
+    __shared__ float4 sl[2][LR * kChunks];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t l0 = (int64_t)(blockIdx.x % lane_tiles) * LR;
+    const int64_t g0 = (int64_t)(blockIdx.x / lane_tiles) * 16 + 4 * wave;
+    const int lrow = MANY ? lane : lane & 15;        // the lane's row of the tile
+    const int lc = tid % kChunks, lr = tid / kChunks;   // the chunk it loads, and its first row (then every kRowStep)
+    const float* lsrc[kLd];
+#pragma unroll
+    for (int i = 0; i < kLd; ++i) lsrc[i] = lanes + min(l0 + lr + kRowStep * i, n_l - 1) * ldl + 4 * lc;
+    const int gk = MANY ? lane >> 2 : lane & 15;     // which of 16 k the lane's group value is, of which group row
+    const float* gsrc = groups + min(g0 + (MANY ? lane & 3 : lane >> 4), n_g - 1) * ldg + gk;
+    f32x4_t acc4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    float acc1 = 0.0f;
+    F4u pre[2][kLd];
+    float gv[2][KS / 16];
+    const int n_full = (int)(n_in / KS);
+    auto load = [&](int step, int slot) {
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) pre[slot][i] = *(const F4u*)(lsrc[i] + (int64_t)step * KS);
+    };
+    auto load_g = [&](int step, int slot) {
+#pragma unroll
+        for (int j = 0; j < KS / 16; ++j) gv[slot][j] = gsrc[(int64_t)step * KS + 16 * j];
+    };
+    auto store = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < kLd; ++i) {
+            const int r = lr + kRowStep * i;
+            const F4u& v = pre[slot][i];
+            sl[slot][r * kChunks + (lc ^ (r & 15))] = make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
+        }
+    };
+    auto products = [&](int slot, int j, float g) {   // k = 16 j .. + 15 of the step in buffer `slot`
+        float b[16];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float4 v = sl[slot][lrow * kChunks + ((4 * j + u) ^ (lrow & 15))];
+            b[4 * u] = v.x, b[4 * u + 1] = v.y, b[4 * u + 2] = v.z, b[4 * u + 3] = v.w;
+        }
+        if constexpr (MANY) mfma16<0>(acc4, g, b);
+        else chain16(acc1, g, b);
+    };
+    // step s from buffer SL; the group values of step s + 1 and the lane values of step s + 2 are issued first (past the
+    // last step: the last one's again, so that no branch holds the loads up)
+    auto step = [&](int s, auto slot_c) {
+        constexpr int SL = decltype(slot_c)::value;
+        lds_barrier();   // (the loads ahead stay in flight)
+        load_g(min(s + 1, n_full - 1), SL ^ 1);
+        load(min(s + 2, n_full - 1), SL);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < KS / 16; ++j) products(SL, j, gv[SL][j]);
+        store(SL ^ 1);   // step s + 1; the buffer's readers (step s - 1) are past this step's barrier
+    };
+    if (n_full > 0) {
+        load(0, 0);
+        load_g(0, 0);
+        load(min(1, n_full - 1), 1);
+        store(0);
+        for (int s = 0; s < n_full; s += 2) {
+            step(s, std::integral_constant<int, 0>{});
+            if (s + 1 >= n_full) break;
+            step(s + 1, std::integral_constant<int, 1>{});
+        }
+    }
+    // the values past the last whole step, and the chain's zeros up to a multiple of 16
+    const int64_t k0 = (int64_t)n_full * KS, left = (n_in + 15) / 16 * 16 - k0;
+    if (left > 0) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kLd; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pre[0][i].v[u] = k0 + 4 * lc + u < n_in ? lsrc[i][k0 + u] : 0.0f;
+        store(0);
+        __syncthreads();
+        for (int j = 0; j < left / 16; ++j) {
+            const int64_t k = k0 + 16 * j;
+            products(0, j, k + gk < n_in ? gsrc[k] : 0.0f);
+        }
+    }
+    if (l0 + lrow >= n_l) return;
+    if constexpr (MANY) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (g0 + i < n_g) y[(l0 + lrow) * yl + (g0 + i) * yg] = acc4[i];
+    } else {
+        if (g0 + (lane >> 4) < n_g) y[(l0 + lrow) * yl + (g0 + (lane >> 4)) * yg] = acc1;
+    }
+}
+
+// The few-chains form up to this many work-groups (16 x 16 chains each, two a compute unit): at 512 (1024 tokens x 128
+// experts x 2048) 20.1 us against 24.5 in 64-row tiles, at 1024 work-groups (2048 tokens) 29.7 against 26.3.
+constexpr int64_t kFewChains = 512;
+// The weight rows lie over the lanes when there are at least as many of them as tokens or a whole tile of 64, so that a
+// logit row's stores are contiguous; else the tokens do (a shared expert's gate is one weight row).
 hipError_t launch_gemm_rows(const float* x, int64_t ldx, const float* w, float* y, int64_t ldy, int64_t n_in,
                             int64_t n_out, int64_t n_tok, hipStream_t s) {
-    const dim3 grid((unsigned)((n_out + kGT - 1) / kGT), (unsigned)((n_tok + kGT - 1) / kGT));
-    hipLaunchKernelGGL(gemm_rows_kernel, grid, dim3(256), 0, s, x, ldx, w, y, ldy, n_in, n_out, n_tok);
+    const bool w_lanes = n_out >= 64 || n_out >= n_tok;
+    const float *pl = w_lanes ? w : x, *pg = w_lanes ? x : w;
+    const int64_t ll = w_lanes ? n_in : ldx, lg = w_lanes ? ldx : n_in, n_l = w_lanes ? n_out : n_tok;
+    const int64_t n_g = w_lanes ? n_tok : n_out, yl = w_lanes ? 1 : ldy, yg = w_lanes ? ldy : 1;
+    const int64_t groups = (n_g + 15) / 16;
+    if ((n_l + 15) / 16 * groups <= kFewChains)
+        hipLaunchKernelGGL(gemm_rows_kernel<false>, dim3((unsigned)((n_l + 15) / 16 * groups)), dim3(256), 0, s, pl, ll,
+                           n_l, pg, lg, n_g, y, yl, yg, n_in, (unsigned)((n_l + 15) / 16));
+    else
+        hipLaunchKernelGGL(gemm_rows_kernel<true>, dim3((unsigned)((n_l + 63) / 64 * groups)), dim3(256), 0, s, pl, ll,
+                           n_l, pg, lg, n_g, y, yl, yg, n_in, (unsigned)((n_l + 63) / 64));
     return hipGetLastError();
 }
 
