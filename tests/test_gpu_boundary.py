@@ -265,3 +265,37 @@ def test_iq_mmq_grouped(xm, t, w_rows, w_cols, counts, use_wtab):
     rel = float((got[:, :w_rows] - ref).abs().max() / ref.abs().max())
     assert rel <= 2e-2, rel
     assert bool((got[:, w_rows:] == 7.0).all())
+
+
+@pytest.mark.parametrize("t,w_rows,w_cols,counts,big", [
+    (8, 256, 256, [1, 31, 0, 33, 128], False), (23, 256, 256, [1, 31, 0, 33, 128], False),
+    (23, 512, 1536, [64, 129, 257, 2, 96], False), (23, 256, 512, [32, 65, 127], True)])
+def test_iq_mmq_grouped_f16_operands(xm, t, w_rows, w_cols, counts, big):
+    """The product of the f16 operands themselves, at the edges of the row tiles: weights rounded to f16 once (IQ4_XS:
+    also codes whose values pass the f16 range, saturated) times activations rounded to f16, against their 64-bit
+    product.  Bound: w_cols fp32 additions of exact products, each rounded to 2^-24 of the running sum of magnitudes."""
+    g = torch.Generator(device=DEV).manual_seed(t + w_cols)
+    n, rb, total = len(counts), xm.row_bytes(t, w_cols), sum(counts)
+    wbuf = torch.zeros(n, (w_rows * rb + 255) // 256 * 256, dtype=torch.uint8, device=DEV)
+    W = []
+    for e in range(n):
+        blk = wbuf[e, :w_rows * rb]
+        xm.quantize_rows(t, torch.randn(w_rows * w_cols, generator=g, device=DEV) * 0.02, out=blk)
+        if big:   # d = 32 and scale 31 in every third block: levels past +-66 pass the f16 range
+            blk.view(-1, 136)[::3, 0:2] = torch.tensor([0x00, 0x50], dtype=torch.uint8, device=DEV)
+            blk.view(-1, 136)[::3, 2:8] = 0xFF
+        w = xm.iq_dequant_f32(t, blk, w_rows * w_cols).reshape(w_rows, w_cols)
+        W.append(w.clamp(-65504, 65504).half().double())
+    bounds = torch.tensor(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), device=DEV)
+    x = torch.randn(total, w_cols, generator=g, device=DEV)
+    xq = xm.iq_mmq_quantize(x, None, w_cols, w_cols, total, True)
+    q = xq[:total * w_cols].view(torch.int8).reshape(total, w_cols).float()
+    d = xq[total * w_cols:total * w_cols + total * (w_cols // 32) * 4].view(torch.float32).reshape(total, -1)
+    a = (q * d.repeat_interleave(32, dim=1)).half().double()
+    ids = torch.arange(total, dtype=torch.int32, device=DEV)
+    dst = torch.zeros(total, w_rows, device=DEV)
+    xm.iq_mmq_grouped(t, wbuf, wbuf.shape[1], w_rows, w_cols, n, xq, total, bounds, ids, dst, w_rows)
+    for e in range(n):
+        r0, r1 = int(bounds[e]), int(bounds[e + 1])
+        want, mag = a[r0:r1] @ W[e].T, a[r0:r1].abs() @ W[e].abs().T
+        assert bool(((dst[r0:r1].double() - want).abs() <= w_cols * 2.0 ** -24 * mag).all()), e

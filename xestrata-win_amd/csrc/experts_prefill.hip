@@ -54,7 +54,7 @@ __host__ __device__ constexpr int lane_rows(bool down, int t) { return down && t
 // row tiles of 32 a work-group: 4 for Q4_K and Q8_0 weights and Q6_K down weights, 2 where the weight words of two
 // rows a lane take more registers (Q6_K gate/up, other formats)
 __host__ __device__ constexpr int row_tiles(bool down, int t) {
-    return t == kQ4_K || t == kQ8_0 || (down && t == kQ6_K) ? 4 : 2;
+    return t == kQ4_K || t == kQ8_0 || t == kIQ4_XS || (down && t == kQ6_K) ? 4 : 2;
 }
 
 // x [n, H] fp32 -> f16 in the step order: thread i writes chunk i (8 values)
@@ -330,7 +330,60 @@ __device__ __forceinline__ f16x8_t q8_frag(const uint4& Q, int kk, uint32_t dbit
     return __builtin_bit_cast(f16x8_t, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
-// ---------------------------------------------------------------- other formats (IQ4_XS, and Q8_0 at other K)
+// ---------------------------------------------------------------- IQ4_XS
+// Step p of a block is sub-blocks 2 p, 2 p + 1 (16 bytes each: values 0 .. 15 the low nibbles, 16 .. 31 the high ones).
+// Lane half hf of a weight row loads sub-block 2 p + hf's 16 bytes; the MFMA order gives it values 16 hf .. + 15 of both
+// sub-blocks, that is the low (hf 0) or high (hf 1) nibbles of both runs, so one v_permlane32_swap of (low nibbles, high
+// nibbles) hands each half its own words of sub-block 2 p (fragments kk 0, 1) and 2 p + 1 (kk 2, 3).  A code's level is
+// two v_perm table reads (levels 0 .. 7 and 8 .. 15, biased by 128 to unsigned bytes) and a third that picks between
+// them; level and scale are multiplied in fp32, where the product is exact ((level + 128) dl - 128 dl: 25 and 24 bits,
+// one fma), and rounded to f16 once, saturating (the kernel sets MODE's FP16_OVFL).  Bound by these ~18 VALU
+// instructions a four codes beside the weight stream; reading each code's byte and level on its own took 5 times as
+// long (hidden 4096, F 1536, 333 tokens: the layer 3,190 -> 656 us; gate/up 2,240, down 944 before).
+struct Iq4Table {
+    uint32_t t[4];
+};
+__device__ __forceinline__ Iq4Table make_iq4_table() {   // kvalues_iq4nl + 128, four a word
+    Iq4Table c;
+    c.t[0] = vreg<0x3F2D1801u>();
+    c.t[1] = vreg<0x766A5D4Fu>();
+    c.t[2] = vreg<0xA6998D81u>();
+    c.t[3] = vreg<0xF1D9C5B5u>();
+    return c;
+}
+__device__ __forceinline__ float iq4_scale(uint2 hdr, int ib) {   // sub-block ib's d (ls - 32)
+    const int ls = (int)((hdr.y >> (4 * ib)) & 0xFu) | (int)(((hdr.x >> (16 + 2 * ib)) & 3u) << 4);
+    return h2f((uint16_t)(hdr.x & 0xFFFFu)) * (float)(ls - 32);
+}
+typedef float f2_t __attribute__((ext_vector_type(2)));
+// four codes (one a byte) -> the f16 pairs (0, 2) and (1, 3)
+__device__ __forceinline__ void iq4_quad(uint32_t n, float dl, float bias, const Iq4Table& tb, uint32_t& p02,
+                                         uint32_t& p13) {
+    const uint32_t m = n & 0x07070707u;
+    const uint32_t lo = __builtin_amdgcn_perm(tb.t[1], tb.t[0], m), hi = __builtin_amdgcn_perm(tb.t[3], tb.t[2], m);
+    const uint32_t v = __builtin_amdgcn_perm(hi, lo, ((n >> 1) & 0x04040404u) | 0x03020100u);
+    float f[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = __builtin_fmaf((float)((v >> (8 * i)) & 0xFFu), dl, bias);
+    p02 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){f[0], f[2]}, h2_t));
+    p13 = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){f[1], f[3]}, h2_t));
+}
+// words (2 i, 2 i + 1) of the lane's run -> fragments kk = i (lo) and i + 2 (hi)
+__device__ __forceinline__ void iq4_frags(uint32_t w0, uint32_t w1, float dl0, float dl1, const Iq4Table& tb, f16x8_t& lo,
+                                          f16x8_t& hi) {
+    const auto a = __builtin_amdgcn_permlane32_swap(w0 & 0x0F0F0F0Fu, (w0 >> 4) & 0x0F0F0F0Fu, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(w1 & 0x0F0F0F0Fu, (w1 >> 4) & 0x0F0F0F0Fu, false, false);
+    const float b0 = -128.0f * dl0, b1 = -128.0f * dl1;
+    uint32_t r[4], q[4];
+    iq4_quad(a[0], dl0, b0, tb, r[0], r[1]);
+    iq4_quad(b[0], dl0, b0, tb, r[2], r[3]);
+    iq4_quad(a[1], dl1, b1, tb, q[0], q[1]);
+    iq4_quad(b[1], dl1, b1, tb, q[2], q[3]);
+    lo = __builtin_bit_cast(f16x8_t, make_uint4(r[0], r[1], r[2], r[3]));
+    hi = __builtin_bit_cast(f16x8_t, make_uint4(q[0], q[1], q[2], q[3]));
+}
+
+// ---------------------------------------------------------------- other formats (mixed layers, and Q8_0 at other K)
 // values [o, o + 8) of the 32-value group g of the block at b, as the reference's host dequantizers give them
 // (dequant.hpp:84-89 Q8_0, 283-299 IQ4_XS)
 __device__ __forceinline__ void dequant8(int type, const uint8_t* b, int g, int o, float (&y)[8]) {
@@ -525,6 +578,7 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
         __syncthreads();
     };
     const QConst qc = make_qconst();
+    if (T == kIQ4_XS) __builtin_amdgcn_s_setreg(1 | (23 << 6), 1);   // MODE.FP16_OVFL: f16 conversions saturate
 
     // The K loop for NRT live row tiles, a compile-time count: a fragment's operand reads and MFMAs are then
     // straight-line code that the scheduler interleaves with the next fragment's dequantization.
@@ -735,6 +789,63 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
             for (int ks = 0; ks < nk; ks += 2) {   // nk is even (K % 128 == 0 for this instance)
                 q8_step(ks, IntC<0>{});
                 q8_step(ks + 1, IntC<1>{});
+            }
+        } else if (T == kIQ4_XS) {
+            // the Q4_K path's pipeline: A rows, the qs runs and (a step before its block) the header of step ks + 1
+            // loaded at the start of step ks with no branch, A written to LDS at its end
+            uint4 areg[RT];
+            auto load_a = [&](int ks) {
+                if (a_live)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i) areg[i] = a_load(i, ks);
+            };
+            auto store_a = [&](int buf) {
+                uint8_t* dst = lds + buf * (kBM * 128) + wave * 8 * RT * 128 + 16 * lane;
+                if (a_live)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i) *(uint4*)(dst + i * 1024) = a_f16(areg[i]);
+            };
+            const Iq4Table tb = make_iq4_table();
+            const int nb = K / 256;
+            uint4 q[2][J];
+            uint2 hdr[J];
+            load_a(0);
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                hdr[j] = ldg8(brow[j]);
+                q[0][j] = ldg16(brow[j] + 8 + 16 * hf);
+            }
+            store_a(0);
+            for (int b = 0; b < nb; ++b) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const int ks = 4 * b + p;
+                    lds_sync();   // A(ks) is in buffer ks & 1; step ks - 1 is done with the other
+                    float dl[J][2];   // first: at p = 3 the header registers take the next block's
+#pragma unroll
+                    for (int j = 0; j < J; ++j) dl[j][0] = iq4_scale(hdr[j], 2 * p), dl[j][1] = iq4_scale(hdr[j], 2 * p + 1);
+                    load_a(min(ks + 1, nk - 1));
+                    const int bn = min(p == 3 ? b + 1 : b, nb - 1);   // the next step's block
+#pragma unroll
+                    for (int j = 0; j < J; ++j) {
+                        const uint8_t* blk = brow[j] + 136 * bn;
+                        if (p == 3) hdr[j] = ldg8(blk);
+                        q[(p + 1) & 1][j] = ldg16(blk + 8 + 32 * ((p + 1) & 3) + 16 * hf);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step's products
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        f16x8_t f0[J], f1[J];
+#pragma unroll
+                        for (int j = 0; j < J; ++j) {
+                            const uint4& D = q[p & 1][j];
+                            iq4_frags(i ? D.z : D.x, i ? D.w : D.y, dl[j][0], dl[j][1], tb, f0[j], f1[j]);
+                        }
+                        mfma_step(ks, i, f0);
+                        mfma_step(ks, i + 2, f1);
+                    }
+                    store_a((ks + 1) & 1);   // after the last step no one reads it
+                }
             }
         } else if constexpr (MMQ) {
             // other formats over MMQ rows: each step's A chunks loaded, converted and written to LDS, then its products
@@ -1191,6 +1302,7 @@ static hipError_t launch_gemm(const ExpertLayout& L, const PrefillArgs& a, hipSt
         t == kQ4_K   ? grouped_mfma_kernel<DOWN, kQ4_K, row_tiles(DOWN, kQ4_K), MMQ>
         : t == kQ6_K ? grouped_mfma_kernel<DOWN, kQ6_K, row_tiles(DOWN, kQ6_K), MMQ>
         : t == kQ8_0 && q8_fast ? grouped_mfma_kernel<DOWN, kQ8_0, row_tiles(DOWN, kQ8_0), MMQ>
+        : t == kIQ4_XS ? grouped_mfma_kernel<DOWN, kIQ4_XS, row_tiles(DOWN, kIQ4_XS), MMQ>
                      : grouped_mfma_kernel<DOWN, 0, row_tiles(DOWN, 0), MMQ>;
     hipLaunchKernelGGL(k, dim3(grid), dim3(256), lds, s, L, a, a.mtile, mt_bound, n_tiles, by_n);
     return hipGetLastError();
