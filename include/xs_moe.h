@@ -6,7 +6,8 @@
  *   - every buffer is device memory owned by the caller; no entry point allocates device memory or synchronises,
  *     except where a NULL stream is allowed and documented to synchronise (the reference's `sync_if_needed`);
  *   - `stream` is a hipStream_t passed as void* (the reference's opaque `void* stream`).  NULL is HIP's ordered default
- *     stream everywhere; the entry points the reference lets run on a null queue then also synchronise.  (The
+ *     stream everywhere; the entry points the reference lets run on a null queue then also synchronise.  HIP's explicit
+ *     handle of the same stream, hipStreamLegacy, enqueues there without that wait.  (The
  *     reference's native router, combine and plan reject a null SYCL queue; the C++ wrappers in
  *     xs_strata_kernels.hpp keep that rule for drop-in callers);
  *   - group and entry counts are read on the device, so one captured graph with capacity grids serves every routing;

@@ -429,3 +429,36 @@ def test_prefill_f16_copy_in_the_permutation_launch(xm):
     assert layer.status() & 8
     with pytest.raises(xm.XsError, match="f16 range"):
         layer.check()
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_default_stream_is_enqueued(xm, shared):
+    """On torch's default stream a prompt layer (its side stream's fork and join included) is enqueued like torch's own
+    operations: the call returns while the stream is still busy, and the output is the one of another stream, bit for
+    bit; so is the raw NULL handle's."""
+    H, E, k, F, T = 1024, 8, 2, 512, 300
+    arena, L = xm.build_arena(E, H, F, xm.Q4_K, xm.Q6_K, seed=3)
+    SL, sh = xm.native_expert_layout(xm.Q8_0, xm.Q8_0, H, F), None
+    if shared:
+        sarena, SL = xm.build_arena(1, H, F, xm.Q8_0, xm.Q8_0, seed=4)
+        sh = (SL, sarena[0], torch.randn(H, device=DEV) * 0.02)
+    layer = xm.MoeLayer(L, arena, E, k, T, prefill=True, shared=sh)
+    x, logits, res = torch.randn(T, H, device=DEV), torch.randn(T, E, device=DEV), torch.randn(T, H, device=DEV)
+    want, out = torch.empty_like(res), torch.empty_like(res)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        layer(x, logits, res, want)
+    torch.cuda.synchronize()
+    sink = torch.zeros(1, dtype=torch.int32, device=DEV)
+    done = torch.cuda.Event()
+    xm._check(xm.lib().xs_bench_occupy(1, 1024, 20_000_000, sink.data_ptr(), xm.STREAM_LEGACY))   # 0.2 s at 100 MHz
+    layer(x, logits, res, out)
+    done.record()
+    assert not done.query()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    out.zero_()
+    layer(x, logits, res, out, stream=0)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)

@@ -32,7 +32,7 @@ int hip_status(hipError_t e, const char* what) {
     if (e != hipSuccess) return fail(XS_EDEVICE, "%s: %s", what, hipGetErrorString(e));
     return ok();
 }
-hipStream_t S(void* s) { return (hipStream_t)s; }
+hipStream_t S(void* s) { return xs::hip_stream(s); }
 // a NULL stream: the default stream, then a wait (the reference's sync_if_needed)
 int finish(void* stream, hipError_t launched, const char* what) {
     if (launched != hipSuccess) return hip_status(launched, what);

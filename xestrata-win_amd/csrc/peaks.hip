@@ -12,6 +12,7 @@
 // decode layer beside other work).
 #include "../../include/xs_moe.h"
 #include "xs_error.h"
+#include "xs_kernels.h"
 
 #include <hip/hip_runtime.h>
 
@@ -116,7 +117,7 @@ extern "C" {
 int xs_bench_hbm_read(const void* src, size_t bytes, unsigned int* sink, int grid, void* stream) {
     if (!src || !sink || ((uintptr_t)src % 16) || bytes % 16 || grid <= 0)
         return xs::set_error(XS_EINVAL, "bench_hbm_read: a span is missing or misaligned, or grid <= 0");
-    hipLaunchKernelGGL(hbm_read_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, (const u32x4*)src,
+    hipLaunchKernelGGL(hbm_read_kernel, dim3((unsigned)grid), dim3(256), 0, xs::hip_stream(stream), (const u32x4*)src,
                        bytes / 16, sink);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? XS_OK : xs::set_error(XS_EDEVICE, std::string("bench_hbm_read: ") + hipGetErrorString(e));
@@ -124,14 +125,14 @@ int xs_bench_hbm_read(const void* src, size_t bytes, unsigned int* sink, int gri
 
 int xs_bench_mfma_f16(int iters, int grid, float* sink, void* stream) {
     if (iters <= 0 || grid <= 0 || !sink) return xs::set_error(XS_EINVAL, "bench_mfma_f16: iters, grid or sink");
-    hipLaunchKernelGGL(mfma_loop_kernel, dim3((unsigned)grid), dim3(128), 0, (hipStream_t)stream, iters, sink);
+    hipLaunchKernelGGL(mfma_loop_kernel, dim3((unsigned)grid), dim3(128), 0, xs::hip_stream(stream), iters, sink);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? XS_OK : xs::set_error(XS_EDEVICE, std::string("bench_mfma_f16: ") + hipGetErrorString(e));
 }
 
 int xs_bench_lds_read(int iters, int grid, unsigned int* sink, void* stream) {
     if (iters <= 0 || grid <= 0 || !sink) return xs::set_error(XS_EINVAL, "bench_lds_read: iters, grid or sink");
-    hipLaunchKernelGGL(lds_read_kernel, dim3((unsigned)grid), dim3(1024), 0, (hipStream_t)stream, iters, sink);
+    hipLaunchKernelGGL(lds_read_kernel, dim3((unsigned)grid), dim3(1024), 0, xs::hip_stream(stream), iters, sink);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? XS_OK : xs::set_error(XS_EDEVICE, std::string("bench_lds_read: ") + hipGetErrorString(e));
 }
@@ -142,7 +143,7 @@ int xs_bench_occupy(int n_wg, int lds_bytes, long long ticks, unsigned int* sink
     hipError_t e = hipFuncSetAttribute((const void*)occupy_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        lds_bytes);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(occupy_kernel, dim3((unsigned)n_wg), dim3(64), (size_t)lds_bytes, (hipStream_t)stream,
+        hipLaunchKernelGGL(occupy_kernel, dim3((unsigned)n_wg), dim3(64), (size_t)lds_bytes, xs::hip_stream(stream),
                            ticks, sink);
         e = hipGetLastError();
     }

@@ -10,6 +10,7 @@
 #include "../../include/xs_tiers.h"
 #include "xs_device.h"
 #include "xs_error.h"
+#include "xs_kernels.h"
 
 #include <hip/hip_runtime.h>
 
@@ -116,7 +117,7 @@ int xs_wait_flag_ge(const uint32_t* flag, uint32_t value, int64_t limit_us, int3
         khz = 100000;
     const long long us = limit_us > 0 ? (limit_us < 3600000000ll ? (long long)limit_us : 3600000000ll) : 10000000ll;
     const long long ticks = us * (long long)khz / 1000;
-    hipLaunchKernelGGL(wait_flag_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, flag, value, ticks, status);
+    hipLaunchKernelGGL(wait_flag_kernel, dim3(1), dim3(64), 0, xs::hip_stream(stream), flag, value, ticks, status);
     return launched(stream, "wait_flag_ge");
 }
 
@@ -126,7 +127,7 @@ int xs_copy_i32_from_mapped(int32_t* dst, const int32_t* src, int64_t n, void* s
     const int vec = a16(dst) && a16(src);
     const int64_t units = vec ? (n + 3) / 4 : n;
     const int groups = (int)std::min<int64_t>(std::max<int64_t>((units + 255) / 256, 1), 64);
-    hipLaunchKernelGGL(copy_i32_mapped_kernel, dim3(groups), dim3(256), 0, (hipStream_t)stream, dst, src, n, vec);
+    hipLaunchKernelGGL(copy_i32_mapped_kernel, dim3(groups), dim3(256), 0, xs::hip_stream(stream), dst, src, n, vec);
     return launched(stream, "copy_i32_from_mapped");
 }
 
@@ -137,7 +138,7 @@ int xs_copy_rows_from_mapped(float* dst, const float* src, int64_t rows, int64_t
         return fail(XS_EINVAL, "copy_rows_from_mapped: width must be a multiple of 4 and both pointers 16-byte aligned");
     if (!hit_rows || !count) return fail(XS_EINVAL, "copy_rows_from_mapped: no hit rows or count");
     if (rows > 0x7fffffff) return fail(XS_EINVAL, "copy_rows_from_mapped: too many rows");
-    hipLaunchKernelGGL(copy_rows_mapped_kernel, dim3((unsigned)rows), dim3(128), 0, (hipStream_t)stream, dst, src, width,
+    hipLaunchKernelGGL(copy_rows_mapped_kernel, dim3((unsigned)rows), dim3(128), 0, xs::hip_stream(stream), dst, src, width,
                        hit_rows, count);
     return launched(stream, "copy_rows_from_mapped");
 }
@@ -151,14 +152,14 @@ int xs_fetch_blobs(const unsigned long long* src, const int32_t* n, uint8_t* dst
     const long long per = blob_bytes / 16;
     // about 512 work-groups in all (two a CU), never more than a blob's words need
     const long long gx = std::max<long long>(1, std::min<long long>((per + 255) / 256, std::max(1, 512 / cap)));
-    hipLaunchKernelGGL(fetch_blobs_kernel, dim3((unsigned)gx, (unsigned)cap), dim3(256), 0, (hipStream_t)stream, src, n,
+    hipLaunchKernelGGL(fetch_blobs_kernel, dim3((unsigned)gx, (unsigned)cap), dim3(256), 0, xs::hip_stream(stream), src, n,
                        (u32x4*)dst, per);
     return launched(stream, "fetch_blobs");
 }
 
 int xs_rebase_ptrs(unsigned long long* ptr, const int32_t* n, uint8_t* base, int64_t blob_bytes, void* stream) {
     if (!ptr || !n) return fail(XS_EINVAL, "rebase_ptrs: no table or count");
-    hipLaunchKernelGGL(rebase_ptrs_kernel, dim3(1), dim3(128), 0, (hipStream_t)stream, ptr, n,
+    hipLaunchKernelGGL(rebase_ptrs_kernel, dim3(1), dim3(128), 0, xs::hip_stream(stream), ptr, n,
                        (unsigned long long)base, (unsigned long long)blob_bytes);
     return launched(stream, "rebase_ptrs");
 }
@@ -169,7 +170,7 @@ int xs_moe_hit_add(float* parts, const float* hit_out, const int32_t* dst, const
     if (!parts || !hit_out || !dst || !count || n_embd <= 0) return fail(XS_EINVAL, "moe_hit_add: no buffer");
     if (cap > 65535) return fail(XS_EINVAL, "moe_hit_add: more than 65535 hits");
     const unsigned gx = (unsigned)std::min<int64_t>((n_embd + 255) / 256, 8);
-    hipLaunchKernelGGL(hit_add_kernel, dim3(gx, (unsigned)cap), dim3(256), 0, (hipStream_t)stream, parts, hit_out, dst,
+    hipLaunchKernelGGL(hit_add_kernel, dim3(gx, (unsigned)cap), dim3(256), 0, xs::hip_stream(stream), parts, hit_out, dst,
                        count, n_embd);
     return launched(stream, "moe_hit_add");
 }

@@ -7,6 +7,11 @@
 
 namespace xs {
 
+// The stream an entry point's handle names.  hipStreamLegacy is the default stream by its explicit handle, which this
+// runtime's event calls do not take (they crash on it); HIP always gets NULL for it here, and only a NULL handed in by
+// the caller makes an entry point wait for the stream.
+inline hipStream_t hip_stream(void* s) { return s == (void*)hipStreamLegacy ? nullptr : (hipStream_t)s; }
+
 struct ExpertLayout {   // one native expert blob: [gate rows | up rows | down rows], raw GGUF blocks
     int gu_type, d_type;
     int64_t n_embd, n_ff;
