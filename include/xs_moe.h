@@ -251,8 +251,8 @@ int xs_add_inplace(float* x, const float* y, int64_t n, void* stream);
  * arena + e * blob_bytes): router -> plan -> q8_1 -> grouped experts -> combine -> residual.
  * out = residual + MoE(x); out may equal residual.  workspace: xs_moe_layer_decode_workspace_bytes for the largest
  * n_tok it will serve, 256-byte aligned, zeroed once before its first call (every call leaves it ready for the next).
- * The layer runs as one persistent launch when n_tok * k <= 256, n_tok <= 64 and the formats are one of Q4_K/Q6_K,
- * Q4_K/Q4_K, Q8_0/Q8_0, IQ4_XS/IQ4_XS; else as the chain of kernels below.  The engine's moe_route + moe_finish
+ * The layer runs as one persistent launch for one token and, below hidden 4096, up to 16 tokens (24 for small layers) of
+ * the formats Q4_K/Q6_K, Q4_K/Q4_K, Q8_0/Q8_0, IQ4_XS/IQ4_XS (n_tok * k <= 256); else as the chain of kernels below.  The engine's moe_route + moe_finish
  * surface (include/strata/core/layer.hpp:108-199) on one GPU, without the host ring. */
 int xs_moe_layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_bytes, int n_expert, int k,
                         const float* x, const float* logits, const float* residual, float* out, int n_tok,

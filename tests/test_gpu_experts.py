@@ -73,6 +73,39 @@ def test_native_expert_grouped(xm, xo, gu, dt, H, F):
     assert int(st[0]) == 0
 
 
+@pytest.mark.parametrize("gu,dt,H,F", [(12, 14, 2048, 768), (12, 12, 1024, 256), (14, 12, 3072, 512), (14, 14, 2048, 256),
+                                       (23, 23, 2048, 512), (23, 8, 1024, 768), (8, 8, 256, 512), (8, 23, 7168, 256)])
+def test_native_expert_grouped_many_entries(xm, xo, gu, dt, H, F):
+    """Groups large enough for the matrix-core rows: 1 to 70 entries a group (one pass of 16 entries, its edges, and
+    passes beyond the four that run side by side), 4 and 8 canonical lanes, every format on either side: the oracle's
+    bits, gate and up rows, h and down rows."""
+    rng = np.random.default_rng(H + F + gu * 100 + dt)
+    arena, L = xm.build_arena(3, H, F, gu, dt, seed=gu + dt)
+    blobs = t2n(arena)
+    sizes, experts, T = [16, 1, 17, 70, 33, 15], [2, 0, 1, 0, 2, 1], 80
+    start, tok, dst = group_case(len(sizes), sizes, T, rng)
+    n = int(start[-1])
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16).float()
+    xq = xm.quantize_q8_1_rows(x.to(DEV))
+    grp_ptr = torch.tensor([arena[e].data_ptr() for e in experts], dtype=torch.int64, device=DEV)
+    ng = torch.tensor([len(sizes)], dtype=torch.int32, device=DEV)
+    scratch = torch.zeros(xm.native_expert_scratch_bytes(n, F), dtype=torch.uint8, device=DEV)
+    out = torch.zeros(n, H, device=DEV)
+    print(f"[case] many entries {gu}/{dt} H={H} F={F}", flush=True)
+    xm.native_expert_grouped(L, grp_ptr, torch.from_numpy(start).to(DEV), ng, torch.from_numpy(dst).to(DEV),
+                             torch.from_numpy(tok).to(DEV), len(sizes), n, xq, scratch, out)
+    torch.cuda.synchronize()
+    want, gate, up, hq = xo.native_expert_grouped(xo.layout(gu, dt, H, F), [blobs[e] for e in experts], start, dst, tok,
+                                                  t2n(xq), n, want_inner=True)
+    fa = (n * F * 4 + 255) & ~255
+    for off, ref in ((0, gate), (fa, up)):
+        got = t2n(scratch[off:off + n * F * 4].view(torch.float32)).reshape(n, F)
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(t2n(scratch[3 * fa:3 * fa + n * (F // 32) * 36]), hq)
+    assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+    assert int(scratch[xm.native_expert_scratch_bytes(n, F) - 256:][:4].view(torch.int32)[0]) == 0
+
+
 def test_grid_groups_same_bits(xm):
     """grid_groups rows of work-groups striding over the groups give the same bits (reference iq_kernels.hpp:85-89)."""
     H, F = 2048, 768

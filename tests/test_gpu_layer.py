@@ -462,3 +462,34 @@ def test_default_stream_is_enqueued(xm, shared):
     layer(x, logits, res, out, stream=0)
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("T,H,F,gu,dt", [(17, 2048, 768, 12, 14), (40, 2048, 768, 12, 14), (2, 4096, 512, 23, 23),
+                                         (12, 4096, 512, 12, 12), (24, 1024, 512, 8, 8), (16, 2048, 768, 12, 14)])
+def test_decode_batch_paths(xm, xo, T, H, F, gu, dt):
+    """The decode layer on either side of its choice of path (one persistent launch up to 16 tokens below hidden 4096,
+    24 for a small layer; else routing, matrix-core rows and combine as launches): the oracle's bits; a batch in which
+    one token's router finds fewer than k experts writes no output and sets bit 2, with or without a good call before
+    it in the same workspace, and the next good call is whole again."""
+    E, k = 16, 8 if H > 1024 else 2
+    arena, L = xm.build_arena(E, H, F, gu, dt, seed=T)
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    logits = torch.randn(T, E, device=DEV, generator=g)
+    x = torch.randn(T, H, device=DEV, generator=g).to(torch.bfloat16).float()
+    res = torch.randn(T, H, device=DEV, generator=g)
+    want = xo.moe_layer_decode(xo.layout(gu, dt, H, F), [t2n(arena[e]) for e in range(E)], k, t2n(x), t2n(logits), t2n(res))
+    layer = xm.MoeLayer(L, arena, E, k, T)
+    bad = logits.clone()
+    bad[T // 2] = float("nan")
+    print(f"[case] batch path T={T} H={H}", flush=True)
+    for lg in (bad, logits, bad, logits):
+        out = torch.full_like(res, 7.0)
+        layer(x, lg, res, out)
+        torch.cuda.synchronize()
+        if lg is bad:
+            assert torch.all(out == 7.0)
+            with pytest.raises(xm.XsError, match="fewer than k experts"):
+                layer.check()
+        else:
+            assert layer.status() == 0
+            assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))

@@ -257,7 +257,11 @@ int grouped_impl(const xs_expert_layout_t* L, const unsigned long long* grp_ptr,
     a.max_entries = max_entries;
     const xs::ExpertLayout XL = to_layout(L);
     hipError_t e;
-    if (xs::stream_usable(XL, max_entries, cap_groups, cap_entries)) {   // the weight-stream kernels (the same bits)
+    // the same bits on each path
+    if (xs::mfma_rows_usable(XL, cap_groups, cap_entries, max_entries)) {   // the units' sums on the matrix cores
+        e = xs::launch_mfma_gu(XL, a, S(stream));
+        if (e == hipSuccess) e = xs::launch_mfma_down(XL, a, S(stream));
+    } else if (xs::stream_usable(XL, max_entries, cap_groups, cap_entries)) {   // the weight-stream kernels
         e = xs::launch_stream_gu(XL, a, S(stream));
         if (e == hipSuccess) e = xs::launch_stream_down(XL, a, S(stream));
     } else {
@@ -939,11 +943,17 @@ int layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_
     const xs::ExpertLayout XL = to_layout(L);
     const bool pre = route.kind == XS_ROUTER_GROUPED_SIGMOID;
     xs::FusedPlan P;
-    // 2..16 tokens of a wide layer (hidden >= 4096): the chained path on the weight-stream kernels, measured faster
-    // there than the persistent layer (config 4 at 8 tokens: 565 -> ~250 us); narrower layers keep the persistent one
-    const bool streamed = n_tok >= 2 && L->n_embd >= 4096 &&
-                          xs::stream_usable(XL, n_tok, capx < n_expert ? capx : n_expert, capx);
-    const bool fused = !streamed && xs::fused_decode_plan(XL, n_expert, k, n_tok, &P);
+    // The chained path (routing, gate/up, h, down, combine) on the matrix-core rows or the weight stream, measured faster
+    // than the persistent layer from 2 tokens of a wide layer on (hidden >= 4096; hidden 4096 IQ4_XS at 8 and 16 tokens
+    // 219 and 394 us against 565 and 502, hidden 7168 Q4_K at 6: 353 against 762) and for more than 16 tokens of a
+    // narrower one (hidden 2048, Q4_K/Q6_K: 17 tokens 135 against 154 us, 24 133 against 195, 32 140 against 239; the
+    // persistent layer stays ahead up to 16: 124 against ~130).  A layer of few, small experts (8 of 1.7 MB, hidden 1024)
+    // is bound by the chain's launches up to ~24 tokens: 20 tokens 39 against 33 us, 24 32 against 39.
+    const int64_t groups = capx < n_expert ? capx : n_expert;
+    const bool rows = xs::mfma_rows_usable(XL, groups, capx, n_tok);
+    const bool chained = L->n_embd >= 4096 ? n_tok >= 2 && (rows || xs::stream_usable(XL, n_tok, groups, capx))
+                                           : rows && (n_tok >= 24 || (n_tok > 16 && groups * (int64_t)L->bytes >= (64 << 20)));
+    const bool fused = !chained && xs::fused_decode_plan(XL, n_expert, k, n_tok, &P);
     // the grouped sigmoid router inside the persistent layer's routing stage where its groups fall on whole lanes
     // (the wave form) and the layout's instances carry it (the Q4_K pair): one launch less (config 5 T=1: 109.5 ->
     // 105.6 us); otherwise its own launch first, into the workspace's ids and weights
@@ -1010,7 +1020,8 @@ int layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_
         // routing, plan and activations in one launch (the reference's router_top10 + resident_plan +
         // quantize_q8_1_rows)
         hipError_t e = xs::launch_decode_route(logits, x, n_tok, n_expert, k, L->n_embd, w.ids, w.w, w.plan, capx,
-                                               w.skip, arena, (long long)blob_bytes, w.xq, S(stream));
+                                               w.skip, arena, (long long)blob_bytes, w.xq, status ? status : w.status,
+                                               S(stream));
         if (e != hipSuccess) return hip_status(e, "moe_layer_decode");
     }
     const int64_t cap_groups = capx < n_expert ? capx : n_expert;
@@ -1019,7 +1030,10 @@ int layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_
     if (int r = grouped_impl(L, (const unsigned long long*)(w.plan + o_ptr), w.plan + o_start, w.plan, w.plan + o_dst,
                              w.plan + o_tok, cap_groups, capx, w.xq, w.scratch, w.parts, stream, 0, n_tok))
         return r;
-    return xs_moe_combine_residual(w.parts, w.w, shared, shared_gate, residual, out, L->n_embd, k, n_tok, stream);
+    // (no output where the routing gave no plan: a token with fewer than k experts, flagged in the status word)
+    return finish(stream, xs::launch_combine(w.parts, w.w, shared, shared_gate, residual, out, L->n_embd, k, n_tok,
+                                             S(stream), w.skip),
+                  "moe_layer_decode");
 }
 }  // namespace
 
@@ -1082,14 +1096,16 @@ int layer_decode_shared(const xs_expert_layout_t* L, const uint8_t* arena, size_
     float* gate = (float*)(base + lw + up256((size_t)n_tok * (size_t)L->n_embd * 4));
     uint8_t* sws = base + lw + up256((size_t)n_tok * (size_t)L->n_embd * 4) + up256((size_t)n_tok * 4);
     const size_t sbytes = shared_ws(SL, n_tok, nullptr).bytes;
-    // up to 64 tokens: the shared expert as a one-expert layer in one persistent launch, in the layer's workspace
+    // up to 16 tokens: the shared expert as a one-expert layer in one persistent launch, in the layer's workspace
     // (its head and tagged words, used again by the routed layer after it) - routing given (expert 0, weight 1.0) and
     // no residual, so each row is the expert's own: fl(y x 1) = y, the canonical rows bit for bit.  That replaces
-    // four launches (q8_1, plan, gate/up, down).  Otherwise, or where the persistent plan does not take the shared
-    // layout or its h would not fit the layer's hand-over region, the shared expert's own chain.
+    // four launches (q8_1, plan, gate/up, down).  Otherwise (64 tokens of hidden 2048, F 768: 55 us against 203 in the
+    // persistent launch), or where the persistent plan does not take the shared layout or its h would not fit the
+    // layer's hand-over region, the shared expert's own chain.
     xs::FusedPlan SP;
     const xs::ExpertLayout SXL = to_layout(SL);
-    if (n_tok <= xs::kOneExpertMaxTok && SL->n_ff <= L->n_ff && fused_possible(L, n_expert, k) &&
+    if ((n_tok <= 16 || (n_tok <= xs::kOneExpertMaxTok && !xs::mfma_rows_usable(SXL, 1, n_tok, n_tok))) &&
+        SL->n_ff <= L->n_ff && fused_possible(L, n_expert, k) &&
         xs::fused_decode_plan(SXL, 1, 1, n_tok, &SP) && aligned(shared_blob, 16)) {
         const DecodeWs w = decode_ws(L, n_expert, k, n_tok, base);
         const int32_t* one_ids = nullptr;

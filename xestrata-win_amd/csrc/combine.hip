@@ -15,10 +15,10 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
                                                       const float* __restrict__ shared,
                                                       const float* __restrict__ shared_gate,
                                                       const float* __restrict__ residual, float* __restrict__ out,
-                                                      int64_t n_embd, int k) {
+                                                      int64_t n_embd, int k, const uint32_t* __restrict__ live) {
     const int64_t t = blockIdx.y;
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n_embd) return;
+    if (c >= n_embd || (live && *live == 0u)) return;
     const float* p = parts + t * k * n_embd + c;
     const float* w = weights + t * k;
     float sum = p[0] * w[0];
@@ -155,10 +155,11 @@ hipError_t launch_combine_h(const uint16_t* parts, const float* weights, const f
 }
 
 hipError_t launch_combine(const float* parts, const float* weights, const float* shared, const float* shared_gate,
-                          const float* residual, float* out, int64_t n_embd, int k, int n_tok, hipStream_t s) {
+                          const float* residual, float* out, int64_t n_embd, int k, int n_tok, hipStream_t s,
+                          const uint32_t* live) {
     const dim3 grid((unsigned)((n_embd + 255) / 256), (unsigned)n_tok);
     hipLaunchKernelGGL(combine_kernel, grid, dim3(256), 0, s, parts, weights, shared, shared_gate, residual, out, n_embd,
-                       k);
+                       k, live);
     return hipGetLastError();
 }
 

@@ -266,6 +266,11 @@ __global__ __launch_bounds__(256) void stream_h_kernel(GroupedArgs a, int F, int
     }
 }
 
+hipError_t launch_stream_h(const ExpertLayout& L, const GroupedArgs& a, int8_t* hq, float* hd, int* hs, hipStream_t s) {
+    hipLaunchKernelGGL(stream_h_kernel, dim3(1024), dim3(256), 0, s, a, (int)L.n_ff, hq, hd, hs);
+    return hipGetLastError();
+}
+
 namespace {
 
 template <bool DOWN>
@@ -363,8 +368,7 @@ hipError_t launch_stream_t(const ExpertLayout& L, const GroupedArgs& a, hipStrea
     float* hd = (float*)(hq + ((f + 255) & ~(size_t)255));
     int* hs = (int*)((uint8_t*)hd + (((f / 32) * 4 + 255) & ~(size_t)255));
     if (DOWN) {
-        hipLaunchKernelGGL(stream_h_kernel, dim3(1024), dim3(256), 0, s, a, (int)L.n_ff, hq, hd, hs);
-        const hipError_t e = hipGetLastError();
+        const hipError_t e = launch_stream_h(L, a, hq, hd, hs, s);
         if (e != hipSuccess) return e;
     }
     switch (canon_lanes(G.n_in / unit)) {

@@ -201,13 +201,12 @@ __device__ __forceinline__ float lane0_sum(float v) {
 }
 
 // bytes of a 16-entry signed table picked by the 4 nibbles of `idx` bytes (each byte < 16): v_perm over the table's
-// halves, then a select on bit 3 of each index
+// halves, then a third that picks each byte from one of them by bit 3 of its index
 __device__ __forceinline__ int table16_lookup(uint32_t idx, uint32_t t0, uint32_t t1, uint32_t t2, uint32_t t3) {
     const uint32_t sel = idx & 0x07070707u;
     const uint32_t lo = __builtin_amdgcn_perm(t1, t0, sel);
     const uint32_t hi = __builtin_amdgcn_perm(t3, t2, sel);
-    const uint32_t m = ((idx & 0x08080808u) >> 3) * 0xFFu;   // 0xFF in every byte whose index is >= 8
-    return (int)((hi & m) | (lo & ~m));
+    return (int)__builtin_amdgcn_perm(hi, lo, ((idx >> 1) & 0x04040404u) | 0x03020100u);
 }
 
 // ---------------------------------------------------------------- 2-byte aligned reads
@@ -248,6 +247,13 @@ __device__ __forceinline__ void dma16_nt(const void* src, uint32_t lds_off) {
 // the same without the nontemporal hint (data other work-groups read again soon)
 __device__ __forceinline__ void dma16(const void* src, uint32_t lds_off) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_off)
+                 : "memory", "m0");
+}
+// dma16_nt from a wave-uniform address and a byte offset a lane.  The base may have been written to its scalar registers
+// by a vector instruction (v_readfirstlane, or the v_readlane of a spill) just before: a vector memory read of them stays
+// five wait states behind, which the compiler does not add inside inline assembly.
+__device__ __forceinline__ void dma16_nt_at(const void* base, uint32_t off, uint32_t lds_off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds_off)
                  : "memory", "m0");
 }
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {

@@ -56,6 +56,13 @@ bool stream_usable(const ExpertLayout& L, int n_tok, int64_t cap_groups, int64_t
 hipError_t launch_stream_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 hipError_t launch_stream_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 
+// h = SwiGLU of the gate/up scratch, per-32 q8 (int8 values, scales, sums of 16; hq's q8_1 blocks too)
+hipError_t launch_stream_h(const ExpertLayout& L, const GroupedArgs& a, int8_t* hq, float* hd, int* hs, hipStream_t s);
+// experts_mfma.hip: the same products with the units' integer sums on the matrix cores (large batches)
+bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries);
+hipError_t launch_mfma_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
+hipError_t launch_mfma_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
+
 // router.hip
 hipError_t launch_router_topk(const float* logits, int n_tokens, int n_expert, int k, int32_t* ids, float* weights,
                               hipStream_t s);
@@ -92,7 +99,7 @@ size_t prefill_route_split_scratch(int64_t n, int n_expert);
 // decode_layer.hip
 hipError_t launch_decode_route(const float* logits, const float* x, int n_tok, int n_expert, int k, int64_t n_embd,
                                int32_t* ids, float* weights, int32_t* plan, long long capx, uint32_t* skip,
-                               const uint8_t* arena, long long blob, void* xq, hipStream_t s);
+                               const uint8_t* arena, long long blob, void* xq, int32_t* err, hipStream_t s);
 
 // decode_fused.hip
 struct FusedPlan {     // the fused decode layer's unit sizes (a function of the layout alone, save ne and lds)
@@ -166,7 +173,8 @@ hipError_t launch_single_group_plan(unsigned long long* grp_ptr, int32_t* start,
 
 // combine.hip
 hipError_t launch_combine(const float* parts, const float* weights, const float* shared, const float* shared_gate,
-                          const float* residual, float* out, int64_t n_embd, int k, int n_tok, hipStream_t s);
+                          const float* residual, float* out, int64_t n_embd, int k, int n_tok, hipStream_t s,
+                          const uint32_t* live = nullptr);   // live: no output when *live is 0
 hipError_t launch_add_inplace(float* x, const float* y, int64_t n, hipStream_t s);
 // the combine over f16 parts, + residual (n_embd % 4 == 0)
 // gemv.hip: the router projections in the reference's summation orders
