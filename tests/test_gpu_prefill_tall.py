@@ -124,3 +124,28 @@ def test_split_under_graph_capture(xm, c3):
         assert torch.equal(out.view(torch.int32), want.view(torch.int32)), i
         other = run_layer(xm, layer, x, logits, res, 0)   # eager work between the replays
         assert torch.equal(other.view(torch.int32), want.view(torch.int32)), i
+
+
+@pytest.mark.parametrize("gu,dt,H,F", [("Q4_K", "Q6_K", 512, 256), ("Q4_K", "Q4_K", 256, 512), ("IQ4_XS", "IQ4_XS", 768, 768),
+                                       ("IQ4_XS", "Q6_K", 1024, 256), ("Q4_K", "IQ4_XS", 2048, 1280)])
+def test_raw_dma_tiles(xm, gu, dt, H, F):
+    """The 128-row GEMMs whose weight words come by DMA (a whole layer's, whose blobs are known to be aligned) against
+    the ones that load them (xs_moe_prefill_experts): the same fragments in the same order, so the layer equals the
+    combine of the standalone parts up to the parts' f16 rounding (half an ulp, 2^-11 of each), at one to five 256-value
+    blocks a row, blocks on and off 16 bytes, and 0, 1, 31, 33, 64, 97, 128, 129 and 200 rows a group."""
+    counts = [0, 1, 31, 33, 64, 97, 128, 129, 200, 15]
+    T, E, k = sum(counts) // 2, len(counts), 2
+    arena, L = xm.build_arena(E, H, F, getattr(xm, gu), getattr(xm, dt), seed=H + F)
+    x, res = inputs(T, H, 11)
+    logits = edge_logits(counts, T, E, 3)
+    print(f"[case] raw dma {gu}/{dt} H={H} F={F}", flush=True)
+    out = run_layer(xm, xm.MoeLayer(L, arena, E, k, T, prefill=True), x, logits, res, 0)
+    ids, w = xm.router_top10(logits, k)
+    r = xm.prefill_route(ids.reshape(-1), k, E, cache_base=arena.data_ptr(), blob=L.bytes, with_ptr=True)
+    parts = torch.zeros(T * k, H, device=DEV)
+    scratch = torch.zeros(xm.moe_prefill_scratch_bytes(T, T * k, H, F), dtype=torch.uint8, device=DEV)
+    xm.moe_prefill_experts(L, x, r["src"], r["entry"], r["bounds"], r["n_groups"], r["grp_ptr"], E, T * k, scratch, parts)
+    parts = parts.reshape(T, k, H).double()
+    want = res.double() + (parts * w[:, :, None].double()).sum(1)
+    lim = 2.0 ** -11 * (parts.abs() * w[:, :, None].double()).sum(1) + 2.0 ** -22 * want.abs() + 1e-7
+    assert bool(((out.double() - want).abs() <= lim).all())

@@ -541,7 +541,7 @@ int prefill_experts(const xs_expert_layout_t* L, const float* x, int64_t n_tok, 
                     const int32_t* entry_of, const int32_t* bounds, const int32_t* n_groups,
                     const unsigned long long* grp_ptr, int64_t cap_groups, int64_t rows, void* scratch, float* parts,
                     uint16_t* parts_h, bool mtile_ready, void* stream, const SideStream* split = nullptr,
-                    int32_t* status = nullptr, bool xb_ready = false) {
+                    int32_t* status = nullptr, bool xb_ready = false, bool blobs16 = false) {
     if (rows <= 0 || cap_groups <= 0) return ok();
     if (int r = check_layout(L, "moe_prefill_experts")) return r;
     if (cap_groups > rows) return fail(XS_EINVAL, "moe_prefill_experts: cap_groups %lld > rows %lld", (long long)cap_groups,
@@ -565,6 +565,7 @@ int prefill_experts(const xs_expert_layout_t* L, const float* x, int64_t n_tok, 
     a.mtile = prefill_mtile(scratch, n_tok, rows, L);
     a.mtile_ready = mtile_ready;
     a.xb_ready = xb_ready;
+    a.blobs16 = blobs16;
     // the f16 saturation bit goes to the caller's status word, else to the scratch's own (xs_moe_prefill_status)
     a.err = status ? status : xs_moe_prefill_status(scratch, n_tok, rows, L->n_embd, L->n_ff);
     a.parts = parts;
@@ -1248,7 +1249,7 @@ int layer_prefill(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob
                            who))
             return r;
         if (int r = prefill_experts(SL, x, n_tok, sw.idx, sw.idx, sw.start, sw.n_groups, sw.grp_ptr, 1, n_tok,
-                                    sw.scratch, sw.rows, nullptr, false, ss, nullptr, w.status))
+                                    sw.scratch, sw.rows, nullptr, false, ss, nullptr, w.status, false, true))
             return r;
         if (w_gate) {
             // the prompt path's gate GEMM order (f32_gemm_rows) at every token count
@@ -1285,7 +1286,7 @@ int layer_prefill(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob
                        who))
         return r;
     if (int r = prefill_experts(L, x, n_tok, w.src, w.entry, w.bounds, w.n_groups, w.grp_ptr, cap_groups, n, w.scratch,
-                                nullptr, w.parts, true, stream, split, w.status, true))
+                                nullptr, w.parts, true, stream, split, w.status, true, true))
         return r;
     if (side)   // the combine waits for the shared expert's rows
         if (hipError_t e = hipStreamWaitEvent(S(stream), side->join, 0)) return hip_status(e, who);

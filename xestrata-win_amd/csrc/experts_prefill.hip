@@ -48,6 +48,12 @@ constexpr int kStageF16 = 128 * 2 + 16, kStageF32 = 128 * 4 + 16;
 constexpr int kStageBytes = 128 * kStageF16 > 64 * kStageF32 ? 128 * kStageF16 : 64 * kStageF32;
 // bytes of LDS before the routing entries of a down tile: the A double buffer or the staging tile, the larger
 __host__ __device__ constexpr int entry_offset(int bm) { return 2 * bm * 128 > kStageBytes ? 2 * bm * 128 : kStageBytes; }
+// the raw-word DMA form: 16-byte chunks of a row's block in LDS (an odd number, so that 16 rows' reads cover the banks; one
+// more than the block's where blocks do not start on 16 bytes), and the LDS bytes before a down tile's routing entries
+__host__ __device__ constexpr int raw_chunks(int t) { return t == kQ4_K ? 9 : t == kQ6_K ? 15 : 11; }
+__host__ __device__ constexpr int raw_entry_offset(int t, int j) {
+    return 2 * 128 * 128 + 4 * 1024 * ((32 * j * raw_chunks(t) + 63) / 64);
+}
 // weight rows a lane dequantizes: one for Q6_K down weights (their raw words take the registers that a 128-row tile
 // needs), two otherwise (gate/up pairs a gate row with its up row)
 __host__ __device__ constexpr int lane_rows(bool down, int t) { return down && t == kQ6_K ? 1 : 2; }
@@ -178,6 +184,12 @@ __device__ __forceinline__ void vm_drain() { asm volatile("s_waitcnt vmcnt(0)" :
 // (__syncthreads() is a release fence too, so it would wait for every load in flight - the prefetch of the steps
 // ahead - before the barrier.)
 __device__ __forceinline__ void lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// wait until at most N of the wave's vector memory operations are outstanding
+template <int N>
+__device__ __forceinline__ void vm_wait_n() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
 
 template <int N>
 struct IntC {
@@ -449,7 +461,7 @@ __device__ __forceinline__ void dma_rows(const uint8_t* const* src, size_t off, 
                                          0);
 }
 
-template <bool DOWN, int T, int RT, bool MMQ = false>
+template <bool DOWN, int T, int RT, bool MMQ = false, bool RAW = false>
 __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, PrefillArgs a,
                                                               const int32_t* __restrict__ mtile, int mt_bound,
                                                               int n_tiles, int by_n) {
@@ -537,7 +549,7 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
         }
     };
     // down: the routing entry of each row, staged in LDS for the epilogue (visible after the first step's barrier)
-    int32_t* const s_entry = (int32_t*)(lds + entry_offset(kBM));
+    int32_t* const s_entry = (int32_t*)(lds + (RAW ? raw_entry_offset(T, J) : entry_offset(kBM)));
     if (DOWN && tid < nrows) s_entry[tid] = a.entry[r0 + tid];
     // the A rows of step ks into buffer `buf`
     auto dma_a = [&](int ks, int buf) {
@@ -600,7 +612,162 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
                 for (int j = 0; j < J; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[i], fb[j], acc[i][j], 0, 0, 0);
         };
-        if (T == kQ4_K) {
+        if constexpr (RAW) {
+            // The raw words by LDS DMA: a wave fetches a whole block (4 steps) of its 32 J rows into its own part of LDS,
+            // 16 bytes a lane along the rows, and takes it into registers when the block begins; the next block's DMA then
+            // goes out in thirds over the block's first steps, behind the A rows of each next step (also by DMA, a step
+            // ahead).  All of it is issued from inline assembly and waited for by count.  Why: a lane's own 16-byte loads
+            // take 32 bytes of each of 32 rows an instruction, and the address and tag lookups of those bound the step-wise
+            // loops (hidden 7168 gate/up: the address unit busy 77% of the kernel's cycles, 31% now, and a quarter fewer
+            // cycles); what bounds it now is the dequantization's and the products' issue, 94% of the cycles together.
+            constexpr int BB = block_bytes(T), NC = raw_chunks(T), NI = (32 * J * NC + 63) / 64;
+            const int nb = K / 256;
+            const uint32_t lds0 = lds_offset(lds), raw0 = lds0 + 2 * kBM * 128 + (uint32_t)wave * (NI * 1024);
+            const uint8_t* const raw = lds + 2 * kBM * 128 + wave * (NI * 1024);
+            // the lane's chunk of DMA instruction i: its row's offset in the blob and the chunk's place in the row's slice.
+            // Lanes past the wave's rows, and a chunk past the slice, fetch the wave's first chunk again.
+            constexpr bool AL16 = BB % 16 == 0;   // (every block on 16 bytes: a lane's address moves by whole blocks)
+            uint32_t roff[NI], rchk[NI];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int idx = 64 * i + lane, r_ = idx / NC, rr = r_ < 32 * J ? r_ : 0;
+                const int jj = rr >> 5, col = (DOWN && J == 2 ? 64 * wave + 32 * jj : 32 * wave) + (rr & 31);   // cb + row
+                const int64_t o = (int64_t)(n0 + col) * wrb + (DOWN ? L.down_off : jj ? L.up_off : 0);
+                rchk[i] = r_ < 32 * J ? (uint32_t)(16 * (idx - r_ * NC)) : 0u;
+                roff[i] = (uint32_t)o + (AL16 ? rchk[i] : 0u);
+            }
+            const uint64_t wp = a.wptr[g];   // (the blob's address in scalar registers; readfirstlane gives an int)
+            const uint8_t* const wblob =
+                (const uint8_t*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(wp >> 32)) << 32) |
+                                 (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)wp));
+            auto dma_raw = [&](int b, int i) {
+                uint32_t at = roff[i];
+                if constexpr (!AL16) {
+                    const uint32_t so = roff[i] + (uint32_t)(BB * b), c = (so & ~15u) + rchk[i];
+                    at = c < so + (uint32_t)BB ? c : so & ~15u;
+                }
+                dma16_at(wblob + (AL16 ? BB * b : 0), at, __builtin_amdgcn_readfirstlane(raw0 + 1024u * i));
+            };
+            const uint8_t* const abase = DOWN ? (const uint8_t*)a.h : (const uint8_t*)a.xb;   // (under 4 GB: the launcher)
+            uint32_t aoff[RT];
+#pragma unroll
+            for (int i = 0; i < RT; ++i) aoff[i] = (uint32_t)(asrc[i] - abase);
+            auto dma_step = [&](int ks, int buf) {   // the A rows that a live row tile reads
+                if (wave < NRT)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i)
+                        dma16_at(abase + (size_t)ks * 128, aoff[i],
+                                 __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(buf * (kBM * 128) +
+                                                                                  (wave * 8 * RT + 8 * i) * 128)));
+            };
+            // the lane's J rows in the wave's part: their bytes keep their address modulo 16
+            const uint8_t* rrow[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) rrow[j] = raw + (32 * j + (lane & 31)) * (NC * 16);
+            struct Raw {   // a block's words of one weight row
+                uint4 q[T == kQ6_K ? 6 : 4], h;   // Q6_K: l0, l1, hq of both halves and the 16 scales
+                uint32_t d;
+            };
+            Raw cur[J];
+            const Iq4Table tb = make_iq4_table();
+            dma_step(0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) dma_raw(0, i);
+            vm_drain();
+            for (int b = 0; b < nb; ++b) {
+#pragma unroll
+                for (int j = 0; j < J; ++j) {   // (brow[j] + BB b: the slice's address)
+                    const int sh = (int)(((uint32_t)(uintptr_t)brow[j] + (uint32_t)(BB * b)) & 15u);
+                    const uint8_t* blk = rrow[j] + sh;
+                    if constexpr (T == kQ4_K) {
+                        cur[j].h = *(const uint4*)rrow[j];
+#pragma unroll
+                        for (int p = 0; p < 4; ++p) cur[j].q[p] = *(const uint4*)(rrow[j] + 16 + 32 * p + 16 * hf);
+                    } else if constexpr (T == kQ6_K) {
+#pragma unroll
+                        for (int n = 0; n < 2; ++n) {
+                            uint32_t w[4];
+                            lds_words_a2<4>(rrow[j], sh + 64 * n + 16 * hf, w);
+                            cur[j].q[3 * n] = make_uint4(w[0], w[1], w[2], w[3]);
+                            lds_words_a2<4>(rrow[j], sh + 64 * n + 32 + 16 * hf, w);
+                            cur[j].q[3 * n + 1] = make_uint4(w[0], w[1], w[2], w[3]);
+                            lds_words_a2<4>(rrow[j], sh + 128 + 32 * n + 16 * hf, w);
+                            cur[j].q[3 * n + 2] = make_uint4(w[0], w[1], w[2], w[3]);
+                        }
+                        uint32_t w[4];
+                        lds_words_a2<4>(rrow[j], sh + 192, w);
+                        cur[j].h = make_uint4(w[0], w[1], w[2], w[3]);
+                        cur[j].d = *(const uint16_t*)(blk + 208);
+                    } else {   // (136 bytes a block: whole 8-byte words)
+                        const uint2 h = *(const uint2*)blk;
+                        cur[j].h.x = h.x, cur[j].h.y = h.y;
+#pragma unroll
+                        for (int p = 0; p < 4; ++p) {
+                            const uint2 w0 = *(const uint2*)(blk + 8 + 32 * p + 16 * hf);
+                            const uint2 w1 = *(const uint2*)(blk + 16 + 32 * p + 16 * hf);
+                            cur[j].q[p] = make_uint4(w0.x, w0.y, w1.x, w1.y);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const int ks = 4 * b + p;
+                    lds_sync();   // A(ks) is in (every wave waited for its rows); step ks - 1 and (p 0) the words are read
+                    dma_step(min(ks + 1, nk - 1), (ks + 1) & 1);
+                    if (p < 3 && b + 1 < nb)
+#pragma unroll
+                        for (int i = p * NI / 3; i < (p + 1) * NI / 3; ++i) dma_raw(b + 1, i);
+                    if constexpr (T == kQ4_K) {
+                        Q4Step sj[J];
+#pragma unroll
+                        for (int j = 0; j < J; ++j) sj[j] = q4k_step(cur[j].h, p);
+#pragma unroll
+                        for (int kk = 0; kk < 4; ++kk) {
+                            f16x8_t fb[J];
+#pragma unroll
+                            for (int j = 0; j < J; ++j) fb[j] = q4k_frag(cur[j].q[p], kk, sj[j], qc);
+                            mfma_step(ks, kk, fb);
+                        }
+                    } else if constexpr (T == kQ6_K) {
+                        const int n = p >> 1, t = p & 1;
+#pragma unroll
+                        for (int kk = 0; kk < 4; ++kk) {
+                            f16x8_t fb[J];
+#pragma unroll
+                            for (int j = 0; j < J; ++j) {
+                                Q6Raw r;
+                                r.l0 = cur[j].q[3 * n], r.l1 = cur[j].q[3 * n + 1], r.hq = cur[j].q[3 * n + 2];
+                                const h2_t sc = q6k_scale_of(n ? make_uint2(cur[j].h.z, cur[j].h.w)
+                                                               : make_uint2(cur[j].h.x, cur[j].h.y), cur[j].d, t, kk, hf);
+                                fb[j] = q6k_frag(r, t, kk, sc, qc);
+                            }
+                            mfma_step(ks, kk, fb);
+                        }
+                    } else {
+                        float dl[J][2];
+#pragma unroll
+                        for (int j = 0; j < J; ++j) {
+                            const uint2 h = make_uint2(cur[j].h.x, cur[j].h.y);
+                            dl[j][0] = iq4_scale(h, 2 * p), dl[j][1] = iq4_scale(h, 2 * p + 1);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            f16x8_t f0[J], f1[J];
+#pragma unroll
+                            for (int j = 0; j < J; ++j) {
+                                const uint4& D = cur[j].q[p];
+                                iq4_frags(i ? D.z : D.x, i ? D.w : D.y, dl[j][0], dl[j][1], tb, f0[j], f1[j]);
+                            }
+                            mfma_step(ks, i, f0);
+                            mfma_step(ks, i + 2, f1);
+                        }
+                    }
+                    // the next step's A rows are in; this step's third of the words may still be on its way
+                    if (p < 3 && b + 1 < nb) vm_wait_n<NI / 3>();
+                    else vm_drain();
+                }
+            }
+        } else if (T == kQ4_K) {
             // The A rows of step ks + 1 go through registers (loaded at the start of step ks, written to LDS at its
             // end), not by LDS DMA: a DMA in flight makes the compiler wait for every load (vmcnt(0)) before the
             // step's first LDS read, which would serialise each step with its own prefetch.
@@ -1289,6 +1456,29 @@ template <bool DOWN, bool MMQ = false>
 static hipError_t launch_gemm(const ExpertLayout& L, const PrefillArgs& a, hipStream_t s, bool rest = false) {
     // (a mixed layer's gate/up: the generic path, which dequantizes each row by its own type)
     const int t = DOWN ? L.d_type : mixed_gu(L) ? -1 : L.gu_type;
+    // The raw words by DMA where every blob is known to start on 16 bytes and offsets fit 32 bits, for the formats of
+    // 256-value blocks (Q6_K: down, whose wave takes 32 rows; not beside the tall tiles, where it measured no faster).
+    // Layers, step-wise loads against it: hidden 7168 Q4_K, 1000 tokens 2,230 -> 1,995 us, 300 tokens 1,727 -> 1,423;
+    // hidden 4096, 333 tokens, IQ4_XS 641 -> 606, Q4_K/Q6_K 627 -> 543; hidden 2048, 100 tokens Q4_K 180 -> 157.
+    if constexpr (!MMQ)
+        if (a.blobs16 && L.bytes < (1ll << 31) && a.n_tok * L.n_embd < (1ll << 31) && a.rows * L.n_ff < (1ll << 31) &&
+            (t == kQ4_K || t == kIQ4_XS || (DOWN && t == kQ6_K && !rest))) {
+            const int J = lane_rows(DOWN, t);
+            const int nt = DOWN ? (int)(L.n_embd / (128 * J)) : (int)(L.n_ff / 128);
+            const int mtb = (int)((a.rows + 127) / 128 + a.cap_groups);
+            const int by_n = nt % 8 == 0 && !rest && !(a.rows < 128 * a.cap_groups);
+            const int lds = raw_entry_offset(t, J) + (DOWN ? 128 * 4 : 0);
+            void (*k)(ExpertLayout, PrefillArgs, const int32_t*, int, int, int) = nullptr;
+            if (t == kQ4_K) k = grouped_mfma_kernel<DOWN, kQ4_K, 4, false, true>;
+            else if (t == kIQ4_XS) k = grouped_mfma_kernel<DOWN, kIQ4_XS, 4, false, true>;
+            else if constexpr (DOWN) k = grouped_mfma_kernel<DOWN, kQ6_K, 4, false, true>;
+            const hipError_t e =
+                hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(k, dim3((unsigned)(by_n ? mtb * nt : 8 * ((mtb + 7) / 8) * nt)), dim3(256), (size_t)lds, s, L,
+                               a, a.mtile, mtb, nt, by_n);
+            return hipGetLastError();
+        }
     const int n_tiles = DOWN ? (int)(L.n_embd / (128 * lane_rows(DOWN, t))) : (int)(L.n_ff / (kBN / 2));
     const bool q8_fast = (DOWN ? L.n_ff : L.n_embd) % 128 == 0;   // Q8_0's own path takes its K steps in pairs
     const int bm = 32 * row_tiles(DOWN, q8_fast ? t : (t == kQ8_0 ? 0 : t));

@@ -256,6 +256,10 @@ __device__ __forceinline__ void dma16_nt_at(const void* base, uint32_t off, uint
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(lds_off)
                  : "memory", "m0");
 }
+__device__ __forceinline__ void dma16_at(const void* base, uint32_t off, uint32_t lds_off) {   // (without the hint)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_off)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }

@@ -205,6 +205,7 @@ hipError_t launch_combine_h(const uint16_t* parts, const float* weights, const f
 
 // experts_prefill.hip
 struct PrefillArgs {
+    bool blobs16 = false;   // every blob is 16-byte aligned (checked by the caller on the host)
     const float* x;                 // [n_tok, n_embd] activations (fp32)
     const int32_t* src;             // [rows] token of each routed row (expert-sorted order)
     const int32_t* entry;           // [rows] routing entry each row writes
