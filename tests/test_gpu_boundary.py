@@ -140,6 +140,22 @@ def test_mmvf_bits(xm, xo, n_tok, n_out, n_in):
     assert np.array_equal(got.view(np.uint32), xo.mmvf(x, wb).view(np.uint32))
 
 
+@pytest.mark.parametrize("n_tok,n_out,n_in", [(1, 3, 2), (1, 2, 66), (2, 3, 960), (5, 3, 1000), (6, 7, 2100),
+                                              (7, 2, 7168), (8, 3, 2560), (1, 5, 16386)])
+def test_mmvf_stride_edges(xm, xo, n_tok, n_out, n_in):
+    """The forms for 1, 2, 4 and 8 tokens where rows end inside four strides (and rows of less than one): the oracle's
+    bits, with x rows further apart than n_in and nothing written past the tokens."""
+    rng = np.random.default_rng(n_in * 8 + n_tok)
+    x = rng.standard_normal((n_tok, n_in)).astype(np.float32)
+    w = (rng.standard_normal((n_out, n_in)) * 0.02).astype(np.float32)
+    wide = torch.full((n_tok, n_in + 6), float("nan"), device=DEV)
+    wide[:, :n_in] = torch.from_numpy(x).to(DEV)
+    y = torch.full((n_tok + 1, n_out), -7.0, device=DEV)
+    xm.f32_gemv_fp32_mmvf_multi(wide[:, :n_in], torch.from_numpy(w).to(DEV), out=y[:n_tok])
+    assert np.array_equal(t2n(y[:n_tok]).view(np.uint32), xo.mmvf(x, w).view(np.uint32))
+    assert (t2n(y[n_tok]) == -7.0).all()
+
+
 @pytest.mark.parametrize("n_tok,n_out,n_in", [(1, 128, 2048), (100, 256, 7168), (300, 128, 2048), (70, 1, 1000),
                                               (9, 65, 48)])
 def test_gemm_rows_bits(xm, xo, n_tok, n_out, n_in):

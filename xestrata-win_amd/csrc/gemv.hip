@@ -65,52 +65,88 @@ __device__ __forceinline__ void weight_pair<uint16_t>(const uint16_t* row, int64
     w1 = u2f(v & 0xFFFF0000u);
 }
 
-template <typename W>
+// sum32 by lane moves inside the VALU: the same additions (after the xor 16 and 8 steps a value repeats every 8 lanes, so
+// a rotation by 4 brings the xor-4 partner's)
+__device__ __forceinline__ float sum32_dpp(float v) {
+    v += swz_xor16_f(v);
+    v += dpp_f<kDppRor8>(v);
+    v += dpp_f<kDppRor4>(v);
+    v += dpp_f<kDppXor2>(v);
+    v += dpp_f<kDppXor1>(v);
+    return v;
+}
+
+// NT: the tokens, rounded up to 1, 2, 4 or 8 (tokens past n_tok repeat the last).  A thread's weight pairs and x values of
+// four strides are in flight together: with one stride's at a time (and the token count a run-time bound) a row waited for
+// memory once a stride, 4 times at 2048 values and 14 at 7168: 1 token x 128 x 2048 5.0 us, now 2.8; 8 tokens x 256 x
+// 7168 39.4, now 13.9.
+template <typename W, int NT>
 __global__ __launch_bounds__(256) void mmvf_kernel(const float* __restrict__ x, int64_t ldx, const W* __restrict__ w,
                                                    float* __restrict__ y, int64_t ldy, int64_t n_pairs, int n_tok) {
-    __shared__ float partials[8 * 32];
+    constexpr int U = 4;
+    __shared__ float partials[NT * 32];
     const int t = threadIdx.x, B = blockDim.x;
     const int64_t o = blockIdx.x;
     const W* row = w + o * 2 * n_pairs;
-    if (B > 32) {
-        if (t < 32)
-            for (int k = 0; k < 8; ++k) partials[k * 32 + t] = 0.0f;
-        __syncthreads();
+    const float* xt[NT];
+    float acc[NT];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        xt[k] = x + min(k, n_tok - 1) * ldx;
+        acc[k] = 0.0f;
     }
-    float acc[8];
+    if (B > 32)
+        for (int i = t; i < NT * 32; i += B) partials[i] = 0.0f;
+    auto strides = [&](int64_t p0, auto whole_c) {   // strides p0, p0 + B, ... (U of them; past the row's end: none)
+        constexpr bool WHOLE = decltype(whole_c)::value;
+        float w0[U], w1[U];
+        float2 xv[U][NT];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] = 0.0f;
-    for (int64_t p = t; p < n_pairs; p += B) {
-        float w0, w1;
-        weight_pair<W>(row, p, w0, w1);
+        for (int u = 0; u < U; ++u) {
+            const int64_t p = WHOLE || p0 + u * B < n_pairs ? p0 + u * B : t;
+            weight_pair<W>(row, p, w0[u], w1[u]);
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (k < n_tok) {
-                const float2 xv = *(const float2*)(x + k * ldx + 2 * p);
-                acc[k] = __builtin_fmaf(w0, xv.x, acc[k]);
-                acc[k] = __builtin_fmaf(w1, xv.y, acc[k]);
-            }
+            for (int k = 0; k < NT; ++k) xv[u][k] = *(const float2*)(xt[k] + 2 * p);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (WHOLE || p0 + u * B < n_pairs)
+#pragma unroll
+                for (int k = 0; k < NT; ++k) {
+                    acc[k] = __builtin_fmaf(w0[u], xv[u][k].x, acc[k]);
+                    acc[k] = __builtin_fmaf(w1[u], xv[u][k].y, acc[k]);
+                }
+    };
+    int64_t p = t;
+    if (t < n_pairs) {
+        for (; p + (U - 1) * B < n_pairs; p += U * B) strides(p, std::true_type{});
+        if (p < n_pairs) strides(p, std::false_type{});
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc[k] = sum32(acc[k]);
+    for (int k = 0; k < NT; ++k) acc[k] = sum32_dpp(acc[k]);
     if (B > 32) {
+        __syncthreads();   // (the zeros are in place)
         if ((t & 31) == 0)
-            for (int k = 0; k < n_tok; ++k) partials[k * 32 + t / 32] = acc[k];
+#pragma unroll
+            for (int k = 0; k < NT; ++k) partials[k * 32 + t / 32] = acc[k];
         __syncthreads();
         if (t < 64) {   // lanes 32..63 run the same sums on the same values; only lane 0 stores
 #pragma unroll
-            for (int k = 0; k < 8; ++k) acc[k] = sum32(partials[k * 32 + (t & 31)]);
+            for (int k = 0; k < NT; ++k) acc[k] = sum32_dpp(partials[k * 32 + (t & 31)]);
         }
     }
     if (t == 0)
-        for (int k = 0; k < n_tok; ++k) y[k * ldy + o] = acc[k];
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+            if (k < n_tok) y[k * ldy + o] = acc[k];
 }
 
 template <typename W>
 hipError_t launch_mmvf(const float* x, int64_t ldx, const W* w, float* y, int64_t ldy, int64_t n_in, int64_t n_out,
                        int n_tok, hipStream_t s) {
-    hipLaunchKernelGGL(mmvf_kernel<W>, dim3((unsigned)n_out), dim3(mmvf_block(n_in)), 0, s, x, ldx, w, y, ldy,
-                       n_in / 2, n_tok);
+    void (*k)(const float*, int64_t, const W*, float*, int64_t, int64_t, int) =
+        n_tok == 1 ? mmvf_kernel<W, 1> : n_tok == 2 ? mmvf_kernel<W, 2> : n_tok <= 4 ? mmvf_kernel<W, 4> : mmvf_kernel<W, 8>;
+    hipLaunchKernelGGL(k, dim3((unsigned)n_out), dim3(mmvf_block(n_in)), 0, s, x, ldx, w, y, ldy, n_in / 2, n_tok);
     return hipGetLastError();
 }
 template hipError_t launch_mmvf<float>(const float*, int64_t, const float*, float*, int64_t, int64_t, int64_t, int,
