@@ -127,12 +127,13 @@ def test_split_under_graph_capture(xm, c3):
 
 
 @pytest.mark.parametrize("gu,dt,H,F", [("Q4_K", "Q6_K", 512, 256), ("Q4_K", "Q4_K", 256, 512), ("IQ4_XS", "IQ4_XS", 768, 768),
-                                       ("IQ4_XS", "Q6_K", 1024, 256), ("Q4_K", "IQ4_XS", 2048, 1280)])
+                                       ("IQ4_XS", "Q6_K", 1024, 256), ("Q4_K", "IQ4_XS", 2048, 1280),
+                                       ("Q8_0", "Q8_0", 256, 384), ("Q8_0", "Q8_0", 1024, 128), ("Q8_0", "Q6_K", 768, 256)])
 def test_raw_dma_tiles(xm, gu, dt, H, F):
     """The 128-row GEMMs whose weight words come by DMA (a whole layer's, whose blobs are known to be aligned) against
     the ones that load them (xs_moe_prefill_experts): the same fragments in the same order, so the layer equals the
     combine of the standalone parts up to the parts' f16 rounding (half an ulp, 2^-11 of each), at one to five 256-value
-    blocks a row, blocks on and off 16 bytes, and 0, 1, 31, 33, 64, 97, 128, 129 and 200 rows a group."""
+    blocks a row (Q8_0: one to eight of 128), blocks on and off 16 bytes, and 0, 1, 31, 33, 64, 97, 128, 129 and 200 rows a group."""
     counts = [0, 1, 31, 33, 64, 97, 128, 129, 200, 15]
     T, E, k = sum(counts) // 2, len(counts), 2
     arena, L = xm.build_arena(E, H, F, getattr(xm, gu), getattr(xm, dt), seed=H + F)

@@ -620,8 +620,11 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
             // take 32 bytes of each of 32 rows an instruction, and the address and tag lookups of those bound the step-wise
             // loops (hidden 7168 gate/up: the address unit busy 77% of the kernel's cycles, 31% now, and a quarter fewer
             // cycles); what bounds it now is the dequantization's and the products' issue, 94% of the cycles together.
-            constexpr int BB = block_bytes(T), NC = raw_chunks(T), NI = (32 * J * NC + 63) / 64;
-            const int nb = K / 256;
+            // (Q8_0: four blocks are one here, 128 values and 136 bytes; 256 values would leave room for one work-group a
+            // compute unit)
+            constexpr int SP = T == kQ8_0 ? 2 : 4;   // steps a block; the next block's DMA goes out over SP - 1 of them
+            constexpr int BB = T == kQ8_0 ? 4 * 34 : block_bytes(T), NC = raw_chunks(T), NI = (32 * J * NC + 63) / 64;
+            const int nb = K / (64 * SP);
             const uint32_t lds0 = lds_offset(lds), raw0 = lds0 + 2 * kBM * 128 + (uint32_t)wave * (NI * 1024);
             const uint8_t* const raw = lds + 2 * kBM * 128 + wave * (NI * 1024);
             // the lane's chunk of DMA instruction i: its row's offset in the blob and the chunk's place in the row's slice.
@@ -665,7 +668,7 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
 #pragma unroll
             for (int j = 0; j < J; ++j) rrow[j] = raw + (32 * j + (lane & 31)) * (NC * 16);
             struct Raw {   // a block's words of one weight row
-                uint4 q[T == kQ6_K ? 6 : 4], h;   // Q6_K: l0, l1, hq of both halves and the 16 scales
+                uint4 q[T == kQ6_K ? 6 : 4], h;   // Q6_K: l0, l1, hq of both halves and the 16 scales; Q8_0: codes, scales
                 uint32_t d;
             };
             Raw cur[J];
@@ -698,6 +701,16 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
                         lds_words_a2<4>(rrow[j], sh + 192, w);
                         cur[j].h = make_uint4(w[0], w[1], w[2], w[3]);
                         cur[j].d = *(const uint16_t*)(blk + 208);
+                    } else if constexpr (T == kQ8_0) {
+                        uint32_t d[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            uint32_t w[4];
+                            lds_words_a2<4>(rrow[j], sh + 34 * i + 2 + 16 * hf, w);
+                            cur[j].q[i] = make_uint4(w[0], w[1], w[2], w[3]);
+                            d[i] = *(const uint16_t*)(blk + 34 * i);
+                        }
+                        cur[j].h = make_uint4(d[0], d[1], d[2], d[3]);
                     } else {   // (136 bytes a block: whole 8-byte words)
                         const uint2 h = *(const uint2*)blk;
                         cur[j].h.x = h.x, cur[j].h.y = h.y;
@@ -710,13 +723,13 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
                     }
                 }
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const int ks = 4 * b + p;
+                for (int p = 0; p < SP; ++p) {
+                    const int ks = SP * b + p;
                     lds_sync();   // A(ks) is in (every wave waited for its rows); step ks - 1 and (p 0) the words are read
                     dma_step(min(ks + 1, nk - 1), (ks + 1) & 1);
-                    if (p < 3 && b + 1 < nb)
+                    if (p < SP - 1 && b + 1 < nb)
 #pragma unroll
-                        for (int i = p * NI / 3; i < (p + 1) * NI / 3; ++i) dma_raw(b + 1, i);
+                        for (int i = p * NI / (SP - 1); i < (p + 1) * NI / (SP - 1); ++i) dma_raw(b + 1, i);
                     if constexpr (T == kQ4_K) {
                         Q4Step sj[J];
 #pragma unroll
@@ -743,6 +756,18 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
                             }
                             mfma_step(ks, kk, fb);
                         }
+                    } else if constexpr (T == kQ8_0) {
+#pragma unroll
+                        for (int kk = 0; kk < 4; ++kk) {
+                            f16x8_t fb[J];
+#pragma unroll
+                            for (int j = 0; j < J; ++j) {
+                                const uint4& D = cur[j].h;
+                                const uint32_t d = p ? (kk >> 1 ? D.w : D.z) : (kk >> 1 ? D.y : D.x);
+                                fb[j] = q8_frag(cur[j].q[2 * p + (kk >> 1)], kk, d, qc);
+                            }
+                            mfma_step(ks, kk, fb);
+                        }
                     } else {
                         float dl[J][2];
 #pragma unroll
@@ -762,8 +787,8 @@ __global__ __launch_bounds__(256, 2) void grouped_mfma_kernel(ExpertLayout L, Pr
                             mfma_step(ks, i + 2, f1);
                         }
                     }
-                    // the next step's A rows are in; this step's third of the words may still be on its way
-                    if (p < 3 && b + 1 < nb) vm_wait_n<NI / 3>();
+                    // the next step's A rows are in; this step's part of the words may still be on its way
+                    if (p < SP - 1 && b + 1 < nb) vm_wait_n<NI / (SP - 1)>();
                     else vm_drain();
                 }
             }
@@ -1456,13 +1481,16 @@ template <bool DOWN, bool MMQ = false>
 static hipError_t launch_gemm(const ExpertLayout& L, const PrefillArgs& a, hipStream_t s, bool rest = false) {
     // (a mixed layer's gate/up: the generic path, which dequantizes each row by its own type)
     const int t = DOWN ? L.d_type : mixed_gu(L) ? -1 : L.gu_type;
-    // The raw words by DMA where every blob is known to start on 16 bytes and offsets fit 32 bits, for the formats of
-    // 256-value blocks (Q6_K: down, whose wave takes 32 rows; not beside the tall tiles, where it measured no faster).
+    // The raw words by DMA where every blob is known to start on 16 bytes and offsets fit 32 bits (Q8_0: whole runs of four
+    // blocks; Q6_K: down, whose wave takes 32 rows; not beside the tall tiles, where it measured no faster).
     // Layers, step-wise loads against it: hidden 7168 Q4_K, 1000 tokens 2,230 -> 1,995 us, 300 tokens 1,727 -> 1,423;
     // hidden 4096, 333 tokens, IQ4_XS 641 -> 606, Q4_K/Q6_K 627 -> 543; hidden 2048, 100 tokens Q4_K 180 -> 157.
+    // Q8_0: hidden 4096, 333 tokens 1,159 -> 637; hidden 2048, 700 tokens 327 -> 229, 4000 849 -> 625; hidden 1024, 65
+    // tokens 54.8 -> 48.9, 700 with a gated shared expert 117.7 -> 111.3.
     if constexpr (!MMQ)
         if (a.blobs16 && L.bytes < (1ll << 31) && a.n_tok * L.n_embd < (1ll << 31) && a.rows * L.n_ff < (1ll << 31) &&
-            (t == kQ4_K || t == kIQ4_XS || (DOWN && t == kQ6_K && !rest))) {
+            (t == kQ4_K || t == kIQ4_XS || (t == kQ8_0 && (DOWN ? L.n_ff : L.n_embd) % 128 == 0) ||
+             (DOWN && t == kQ6_K && !rest))) {
             const int J = lane_rows(DOWN, t);
             const int nt = DOWN ? (int)(L.n_embd / (128 * J)) : (int)(L.n_ff / 128);
             const int mtb = (int)((a.rows + 127) / 128 + a.cap_groups);
@@ -1471,6 +1499,7 @@ static hipError_t launch_gemm(const ExpertLayout& L, const PrefillArgs& a, hipSt
             void (*k)(ExpertLayout, PrefillArgs, const int32_t*, int, int, int) = nullptr;
             if (t == kQ4_K) k = grouped_mfma_kernel<DOWN, kQ4_K, 4, false, true>;
             else if (t == kIQ4_XS) k = grouped_mfma_kernel<DOWN, kIQ4_XS, 4, false, true>;
+            else if (t == kQ8_0) k = grouped_mfma_kernel<DOWN, kQ8_0, 4, false, true>;
             else if constexpr (DOWN) k = grouped_mfma_kernel<DOWN, kQ6_K, 4, false, true>;
             const hipError_t e =
                 hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
