@@ -184,7 +184,10 @@ __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom 
                     for (int r = 0; r < 4; ++r) acc[c][r] = 0.0f;
                 for (int st = 0; st < G.steps; ++st, ++q) {
                     {
-                        if (q + G.slots - 1 < total) issue();
+                        if (q + G.slots - 1 < total) {   // into the slot that the last step read
+                            lds_reads_done();
+                            issue();
+                        }
                         vm_wait_le(min(G.slots - 1, total - 1 - q) * G.ni);
                         const uint8_t* const slot = ring + c_slot;
                         c_slot = c_slot + slot_bytes == ring_end - ring_lds ? 0u : c_slot + slot_bytes;

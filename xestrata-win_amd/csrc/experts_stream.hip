@@ -139,6 +139,7 @@ __global__ __launch_bounds__(64 * WAVES) void stream_kernel(GroupedArgs a, Strea
         const int r0_ = i_rg * G.R;
         const int so0 = (int)G.mat_off + r0_ * G.rb + i_s * G.segb;
         const uint32_t slot_off = ring_off + (uint32_t)((q % G.slots) * G.slot);
+        lds_reads_done();   // (the slot's last readers among them)
 #pragma unroll
         for (int j = 0; j < kStreamNiMax; ++j) {
             if (j >= G.ni) break;

@@ -260,6 +260,9 @@ __device__ __forceinline__ void dma16_at(const void* base, uint32_t off, uint32_
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_off)
                  : "memory", "m0");
 }
+// Before a DMA into a slot of a ring that this wave has read: its LDS reads have returned.  A DMA takes no part in lgkmcnt,
+// and what a read is used for, with the compiler's own wait, may come after the DMA in the code.
+__device__ __forceinline__ void lds_reads_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
