@@ -686,7 +686,7 @@ __global__ __launch_bounds__(fused_threads(NE, MODE)) void moe_decode_fused_kern
                     for (int e = 0; e < NE; ++e) acc[e] = 0.0f;
                     const uint8_t* rb = row_base(rr);
                     for (int u = c; u < H / UG::kUnit; u += lpr_g)
-                        UG::template apply<NE>(rb, rr * (int)L.gu_row, u, actg, m, acc);
+                        UG::template apply<NE, DIRECT>(rb, rr * (int)L.gu_row, u, actg, m, acc);
 #pragma unroll
                     for (int e = 0; e < NE; ++e) acc[e] = lanes_sum(acc[e], lpr_g);
                     if (c == 0) {
@@ -781,7 +781,7 @@ __global__ __launch_bounds__(fused_threads(NE, MODE)) void moe_decode_fused_kern
 #pragma unroll
                         for (int e = 0; e < M; ++e) acc[e] = 0.0f;
                         for (int u = c; u < F / UD::kUnit; u += lpr_d)
-                            UD::template apply<M>(rb, rr * (int)L.d_row, u, am, M, acc);
+                            UD::template apply<M, DIRECT>(rb, rr * (int)L.d_row, u, am, M, acc);
 #pragma unroll
                         for (int e = 0; e < M; ++e) acc[e] = lanes_sum(acc[e], lpr_d);
                         if (c == 0) {

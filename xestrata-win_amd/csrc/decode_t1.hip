@@ -230,7 +230,7 @@ __device__ __forceinline__ void t1_help_unit(const uint8_t* arena, long long blo
                                      : blob + up_off + (size_t)(32 * j + rr - 32) * gu_row;
         float acc[1] = {0.0f};
         const Act at[1] = {ax};
-        for (int u = c; u < H / UG::kUnit; u += lprc) UG::template apply<1>(row, 0, u, at, 1, acc);
+        for (int u = c; u < H / UG::kUnit; u += lprc) UG::template apply<1, true>(row, 0, u, at, 1, acc);
         const float sm = lane0_sum<lprc>(acc[0]);
         if (c == 0) s_gu[rr] = sm;
     }

@@ -50,12 +50,26 @@ __device__ __forceinline__ void lds_words_a2(const uint8_t* base, int off, uint3
 #pragma unroll
     for (int i = 0; i < NW; ++i) w[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], sh);
 }
+// the same from global memory: nothing past the last word that holds a wanted byte is read (where the bytes start on a word
+// that is word NW - 1, and word NW may lie past the end of the allocation)
+template <int NW>
+__device__ __forceinline__ void global_words_a2(const uint8_t* base, int off, uint32_t (&w)[NW]) {
+    const uint32_t* q = (const uint32_t*)(base + (off & ~3));
+    const uint32_t sh = (uint32_t)(off & 3);
+    uint32_t d[NW + 1];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) d[i] = q[i];
+    d[NW] = q[sh ? NW : NW - 1];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) w[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], sh);
+}
 
 __device__ __forceinline__ int us32(const Act& a, int g) { return a.us16[2 * g] + a.us16[2 * g + 1]; }
 
 // PAD: bytes between the int8 values of consecutive 256-value blocks of the activation (0: packed).  Lanes of a row
 // read the same piece of 8 neighbouring blocks at once; 256 bytes apart those reads all hit the same LDS banks, 272
 // apart they spread over all of them.
+// apply's GLOBAL: the rows are in global memory, where nothing past a row's last word may be read.
 template <int T, bool S256, int PAD = 0>
 struct Unit;
 // the padding the modular kernels give their staged gate/up rows, and a staged row's int8 bytes with a padding
@@ -66,7 +80,7 @@ __host__ __device__ inline int act_rowq(int n, int pad) { return n + ((n + 255) 
 template <bool S256, int PAD>
 struct Unit<kQ4_K, S256, PAD> {
     static constexpr int kUnit = S256 ? 256 : 32;
-    template <int NE>
+    template <int NE, bool GLOBAL = false>
     __device__ static __forceinline__ void apply(const uint8_t* base, int roff, int u, const Act (&a)[NE], int n,
                                                  float (&acc)[NE]) {
         const int b = S256 ? u : u >> 3;
@@ -170,7 +184,7 @@ struct Unit<kQ6_K, S256, PAD> {
             S[e] += sc0 * i0 + sc1 * i1;
         }
     }
-    template <int NE>
+    template <int NE, bool GLOBAL = false>
     __device__ static __forceinline__ void apply(const uint8_t* base, int roff, int u, const Act (&a)[NE], int n,
                                                  float (&acc)[NE]) {
         const int b = S256 ? u : u >> 3;
@@ -197,13 +211,14 @@ struct Unit<kQ6_K, S256, PAD> {
 template <bool S256, int PAD>
 struct Unit<kQ8_0, S256, PAD> {
     static constexpr int kUnit = 32;
-    template <int NE>
+    template <int NE, bool GLOBAL = false>
     __device__ static __forceinline__ void apply(const uint8_t* base, int roff, int u, const Act (&a)[NE], int n,
                                                  float (&acc)[NE]) {
         const int boff = roff + 34 * u;
         const float d = h2f(*(const uint16_t*)(base + boff));
         uint32_t w[8];
-        lds_words_a2<8>(base, boff + 2, w);
+        if (GLOBAL) global_words_a2<8>(base, boff + 2, w);   // (its last byte is the block's last, and the blob's)
+        else lds_words_a2<8>(base, boff + 2, w);
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
             if (e >= n) break;
@@ -254,7 +269,7 @@ struct Unit<kIQ4_XS, S256, PAD> {
             S[e] += ls * is;
         }
     }
-    template <int NE>
+    template <int NE, bool GLOBAL = false>
     __device__ static __forceinline__ void apply(const uint8_t* base, int roff, int u, const Act (&a)[NE], int n,
                                                  float (&acc)[NE]) {
         const int b = S256 ? u : u >> 3;
