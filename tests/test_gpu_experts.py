@@ -215,3 +215,25 @@ def test_prefill_experts_saturation_status(xm):
             with pytest.raises(xm.XsError, match="f16 range"):
                 xm._check(xm.lib().xs_moe_status_check(status, None))
         xm._check(xm.lib().xs_moe_status_check(status, None))   # clear (again)
+
+
+@pytest.mark.parametrize("T", [2, 3, 4, 5])
+@pytest.mark.parametrize("gu,H,F", [(8, 2048, 640), (8, 2048, 1408), (12, 2048, 1408), (8, 4096, 384), (8, 4096, 1536)])
+def test_q8_0_down_of_several_steps(xm, xo, gu, H, F, T):
+    """Q8_0 down rows that the weight stream takes in several steps (F 640: 5, F 1408: 11 at up to 4 tokens), beside
+    one-step rows (F 384), more tokens, and F 1536, whose rows took two steps before the matrix-core rows: the shared
+    expert's rows and the layer's output (hidden 4096: the stream's layers) are the oracle's bits."""
+    E, k = 4, 2
+    arena, L = xm.build_arena(E, H, F, gu, 8, seed=F + T)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, H, device=DEV, generator=g).to(torch.bfloat16).float()
+    logits, res = torch.randn(T, E, device=DEV, generator=g), torch.randn(T, H, device=DEV, generator=g)
+    print(f"[case] q8_0 down steps gu={gu} H={H} F={F} T={T}", flush=True)
+    ol, blobs = xo.layout(gu, 8, H, F), [t2n(arena[e]) for e in range(E)]
+    rows, _ = xm.shared_expert_decode(L, arena[1], x)
+    assert np.array_equal(t2n(rows).view(np.uint32), xo.shared_expert(ol, blobs[1], t2n(x)).view(np.uint32))
+    layer, out = xm.MoeLayer(L, arena, E, k, T), torch.empty_like(res)
+    layer(x, logits, res, out)
+    want = xo.moe_layer_decode(ol, blobs, k, t2n(x), t2n(logits), t2n(res), n_threads=8)
+    assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+    assert layer.status() == 0

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(64 * WAVES) void stream_kernel(GroupedArgs a, Strea
                     ws16[e * nb16 + k] = hact_s[(int64_t)(e0 + p0 + e) * nb16 + k];
                 }
             }
-            if (DOWN || s == 0 || npass > 1) {
+            if (s == 0 || npass > 1) {   // (a task of several steps keeps its chains over them)
 #pragma unroll
                 for (int e = 0; e < NE; ++e) {
                     acc[e] = 0.0f;
