@@ -237,3 +237,33 @@ def test_q8_0_down_of_several_steps(xm, xo, gu, H, F, T):
     want = xo.moe_layer_decode(ol, blobs, k, t2n(x), t2n(logits), t2n(res), n_threads=8)
     assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
     assert layer.status() == 0
+
+
+@pytest.mark.parametrize("H,F,sizes", [(256, 512, [1, 16, 17]), (2048, 256, [5, 2]), (4096, 256, [70, 1]), (7168, 512, [16, 3])])
+def test_native_expert_grouped_scale_a_block(xm, xo, H, F, sizes):
+    """q8_1 rows with a scale of its own in each 32-value block, as a caller's quantizer may give them, for Q8_0 gate/up
+    rows: the whole call and its two halves are the oracle's bits (each block's own scale counts)."""
+    rng = np.random.default_rng(H + F)
+    arena, L = xm.build_arena(2, H, F, 8, 8, seed=H)
+    start, tok, dst = group_case(len(sizes), sizes, 20, rng)
+    n, experts = int(start[-1]), [i % 2 for i in range(len(sizes))]
+    x = rng.standard_normal((20, H)).astype(np.float32) * np.exp(rng.standard_normal((20, H // 32, 1)).repeat(32, 2)
+                                                                 .reshape(20, H)).astype(np.float32)
+    xq = xo.quantize_q8_1_per32(x)
+    dx, d_start, d_tok, d_dst = (torch.from_numpy(v).to(DEV) for v in (xq, start, tok, dst))
+    grp_ptr = torch.tensor([arena[e].data_ptr() for e in experts], dtype=torch.int64, device=DEV)
+    ng = torch.tensor([len(sizes)], dtype=torch.int32, device=DEV)
+    print(f"[case] scale a block H={H} F={F}", flush=True)
+    outs = []
+    for whole in (True, False):
+        scratch = torch.zeros(xm.native_expert_scratch_bytes(n, F), dtype=torch.uint8, device=DEV)
+        out = torch.zeros(n, H, device=DEV)
+        if whole:
+            xm.native_expert_grouped(L, grp_ptr, d_start, ng, d_dst, d_tok, len(sizes), n, dx, scratch, out)
+        else:
+            xm.native_expert_gate_up(L, grp_ptr, d_start, ng, d_tok, len(sizes), n, dx, scratch)
+            xm.native_expert_down(L, grp_ptr, d_start, ng, d_dst, len(sizes), n, scratch, out)
+        outs.append(t2n(out))
+    want = xo.native_expert_grouped(xo.layout(8, 8, H, F), [t2n(arena[e]) for e in experts], start, dst, tok, xq, n)
+    for got in outs:
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))

@@ -243,11 +243,12 @@ int grouped_args(const xs_expert_layout_t* L, const unsigned long long* grp_ptr,
     return ok();
 }
 
-// max_entries: the most entries one group can hold (the call's token count), 0 when not known
+// max_entries: the most entries one group can hold (the call's token count), 0 when not known.  own_rows: x_q8_1 is from
+// quantize_q8_1_rows, one scale repeated over 256 values
 int grouped_impl(const xs_expert_layout_t* L, const unsigned long long* grp_ptr, const int32_t* grp_start,
                  const int32_t* n_groups, const int32_t* ent_dst, const int32_t* ent_tok, int64_t cap_groups,
                  int64_t cap_entries, const void* x_q8_1, void* scratch, float* out, void* stream, int64_t grid_groups,
-                 int max_entries) {
+                 int max_entries, bool own_rows) {
     if (cap_groups <= 0 || cap_entries <= 0) return ok();
     if (!ent_dst || !ent_tok || !x_q8_1 || !out) return fail(XS_EINVAL, "native_expert_grouped: a span is missing");
     xs::GroupedArgs a;
@@ -255,10 +256,11 @@ int grouped_impl(const xs_expert_layout_t* L, const unsigned long long* grp_ptr,
                              scratch, out, grid_groups, "native_expert_grouped", &a))
         return r;
     a.max_entries = max_entries;
+    a.x_scale32 = !own_rows;
     const xs::ExpertLayout XL = to_layout(L);
     hipError_t e;
     // the same bits on each path
-    if (xs::mfma_rows_usable(XL, cap_groups, cap_entries, max_entries)) {   // the units' sums on the matrix cores
+    if (xs::mfma_rows_usable(XL, cap_groups, cap_entries, max_entries, !own_rows)) {   // the units' sums on the matrix cores
         e = xs::launch_mfma_gu(XL, a, S(stream));
         if (e == hipSuccess) e = xs::launch_mfma_down(XL, a, S(stream));
     } else if (xs::stream_usable(XL, max_entries, cap_groups, cap_entries)) {   // the weight-stream kernels
@@ -277,7 +279,7 @@ int xs_native_expert_grouped(const xs_expert_layout_t* L, const unsigned long lo
                              const int32_t* ent_tok, int64_t cap_groups, int64_t cap_entries, const void* x_q8_1,
                              void* scratch, float* out, void* stream, int64_t grid_groups) {
     return grouped_impl(L, grp_ptr, grp_start, n_groups, ent_dst, ent_tok, cap_groups, cap_entries, x_q8_1, scratch,
-                        out, stream, grid_groups, 0);
+                        out, stream, grid_groups, 0, false);
 }
 
 int xs_native_expert_gate_up(const xs_expert_layout_t* L, const unsigned long long* grp_ptr, const int32_t* grp_start,
@@ -749,7 +751,7 @@ int xs_shared_expert_decode(const xs_expert_layout_t* SL, const uint8_t* blob, c
                        "shared_expert_decode"))
         return r;
     if (int r = grouped_impl(SL, w.grp_ptr, w.start, w.n_groups, w.idx, w.idx, 1, n_tok, w.xq, w.scratch, shared,
-                             stream, 0, n_tok))
+                             stream, 0, n_tok, true))
         return r;
     if (w_gate) return xs_router_logits_f32(x, w_gate, gate_logit, n_tok, SL->n_embd, 1, stream);
     return ok();
@@ -1029,7 +1031,7 @@ int layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_
     long long o_start, o_dst, o_tok, o_ptr;
     xs_plan_offsets(capx, &o_start, &o_dst, &o_tok, &o_ptr, nullptr);
     if (int r = grouped_impl(L, (const unsigned long long*)(w.plan + o_ptr), w.plan + o_start, w.plan, w.plan + o_dst,
-                             w.plan + o_tok, cap_groups, capx, w.xq, w.scratch, w.parts, stream, 0, n_tok))
+                             w.plan + o_tok, cap_groups, capx, w.xq, w.scratch, w.parts, stream, 0, n_tok, true))
         return r;
     // (no output where the routing gave no plan: a token with fewer than k experts, flagged in the status word)
     return finish(stream, xs::launch_combine(w.parts, w.w, shared, shared_gate, residual, out, L->n_embd, k, n_tok,

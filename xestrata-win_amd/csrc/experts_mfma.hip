@@ -59,7 +59,10 @@ __host__ __device__ constexpr int mfma_step_blocks(int t, bool down) {
     return t == kQ8_0 ? 8 : down || t == kQ6_K ? 1 : 2;
 }
 
-template <int T, bool DOWN, int L>
+// X32 (Q8_0 gate/up): the q8_1 rows have a scale of their own in each 32-value block, kept as the fp16 it comes in (hidden
+// 7168: 16 entries still fit beside the rings).  Rows of quantize_q8_1_rows repeat one scale over 256 values, which is
+// read once a step (16 tokens of hidden 7168: 676 us a layer against 711 with a read a block).
+template <int T, bool DOWN, int L, bool X32>
 __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom G, const int8_t* __restrict__ hq,
                                                         const float* __restrict__ hd) {
     constexpr int SB = mfma_step_blocks(T, DOWN), BB = block_bytes(T);
@@ -69,7 +72,8 @@ __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = 64 * G.waves;
     const int lrow = lane & 15, oct = lane >> 4;          // the lane's weight row (and entry of A), its octet of 32 values
     uint8_t* const aq = lds;
-    float* const ad = (float*)(lds + G.ent * G.astride);   // [scale][entry]: one scale a 256 (gate/up) or 32 (down)
+    static_assert(!X32 || (T == kQ8_0 && !DOWN));
+    float* const ad = (float*)(lds + G.ent * G.astride);   // [scale][entry]: one scale a 256 (gate/up) or 32 (down; X32: fp16)
     uint8_t* const ring = lds + G.ring_off + wave * (G.slots * G.ni * 1024);
     const uint32_t ring_lds = lds_offset(ring);
     const uint32_t iq_t[4] = {kIq4Tab[0], kIq4Tab[1], kIq4Tab[2], kIq4Tab[3]};
@@ -142,7 +146,8 @@ __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom 
                     uint4* dst = (uint4*)(aq + e * G.astride + 32 * bi);
                     dst[0] = make_uint4(w[1], w[2], w[3], w[4]);
                     dst[1] = make_uint4(w[5], w[6], w[7], w[8]);
-                    if ((bi & 7) == 0) ad[(bi >> 3) * kMfmaEnt + e] = h2f((uint16_t)(w[0] & 0xFFFFu));
+                    if (X32) ((uint16_t*)ad)[bi * kMfmaEnt + e] = (uint16_t)(w[0] & 0xFFFFu);
+                    else if ((bi & 7) == 0) ad[(bi >> 3) * kMfmaEnt + e] = h2f((uint16_t)(w[0] & 0xFFFFu));
                 }
             } else {
                 const int nc16 = G.n_in >> 4;
@@ -201,7 +206,14 @@ __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom 
                                 lds_words_a2<2>(slot, roff + 34 * c + 2 + 8 * oct, w);
                                 const float d = h2f(*(const uint16_t*)(slot + roff + 34 * c));
                                 const i32x4_t D = mfma(act(u), codes8(w[0], w[1]), zero);
-                                const float4 d8 = *(const float4*)(adl + (DOWN ? u : st) * kMfmaEnt);
+                                float4 d8;
+                                if (X32) {
+                                    const uint2 h = *(const uint2*)((const uint16_t*)ad + u * kMfmaEnt + 4 * oct);
+                                    d8 = make_float4(h2f((uint16_t)(h.x & 0xFFFFu)), h2f((uint16_t)(h.x >> 16)),
+                                                     h2f((uint16_t)(h.y & 0xFFFFu)), h2f((uint16_t)(h.y >> 16)));
+                                } else {
+                                    d8 = *(const float4*)(adl + (DOWN ? u : st) * kMfmaEnt);
+                                }
                                 acc[c][0] = __builtin_fmaf(d * d8.x, (float)D[0], acc[c][0]);
                                 acc[c][1] = __builtin_fmaf(d * d8.y, (float)D[1], acc[c][1]);
                                 acc[c][2] = __builtin_fmaf(d * d8.z, (float)D[2], acc[c][2]);
@@ -364,7 +376,7 @@ __global__ __launch_bounds__(512) void rows_mfma_kernel(GroupedArgs a, MfmaGeom 
 namespace {
 
 template <int T, bool DOWN>
-bool mfma_geom(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries, MfmaGeom& G) {
+bool mfma_geom(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries, bool x32, MfmaGeom& G) {
     constexpr int SB = mfma_step_blocks(T, DOWN), BB = block_bytes(T), BV = block_values(T);
     G.n_in = (int)(DOWN ? L.n_ff : L.n_embd);
     G.rows_total = (int)(DOWN ? L.n_embd : 2 * L.n_ff);
@@ -380,7 +392,7 @@ bool mfma_geom(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, i
     G.ni = (16 * G.nc + 63) / 64;
     if (G.ni > kMfmaNi) return false;
     G.astride = G.n_in + 32;
-    const int scales = (DOWN ? G.n_in / 32 : G.n_in / 256) * kMfmaEnt * 4;
+    const int scales = DOWN ? G.n_in / 32 * kMfmaEnt * 4 : x32 ? G.n_in / 32 * kMfmaEnt * 2 : G.n_in / 256 * kMfmaEnt * 4;
     G.ent = max_entries > 0 && max_entries < kMfmaEnt ? (int)max_entries : kMfmaEnt;
     G.ring_off = (G.ent * G.astride + scales + 15) & ~15;
     // work-groups of 4 waves, two or more a compute unit (one starts, its indices and activations on their way, while
@@ -402,9 +414,9 @@ bool mfma_geom(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, i
     return true;
 }
 
-template <int T, bool DOWN, int LC>
+template <int T, bool DOWN, int LC, bool X32 = false>
 hipError_t launch_one(const GroupedArgs& a, const MfmaGeom& G, const int8_t* hq, const float* hd, hipStream_t s) {
-    void (*kern)(GroupedArgs, MfmaGeom, const int8_t*, const float*) = rows_mfma_kernel<T, DOWN, LC>;
+    void (*kern)(GroupedArgs, MfmaGeom, const int8_t*, const float*) = rows_mfma_kernel<T, DOWN, LC, X32>;
     const int lds = G.ring_off + G.waves * G.slots * G.ni * 1024;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -423,7 +435,8 @@ hipError_t launch_one(const GroupedArgs& a, const MfmaGeom& G, const int8_t* hq,
 template <int T, bool DOWN>
 hipError_t launch_t(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) {
     MfmaGeom G;
-    if (!mfma_geom<T, DOWN>(L, a.cap_groups, a.cap_entries_hint, a.max_entries, G)) return hipErrorNotSupported;
+    const bool x32 = a.x_scale32 && !DOWN && T == kQ8_0;
+    if (!mfma_geom<T, DOWN>(L, a.cap_groups, a.cap_entries_hint, a.max_entries, x32, G)) return hipErrorNotSupported;
     const size_t f = (size_t)a.cap_entries_hint * (size_t)L.n_ff;   // the h region: int8 values, scales, sums of 16
     int8_t* hq = (int8_t*)a.hact;
     float* hd = (float*)(hq + ((f + 255) & ~(size_t)255));
@@ -439,31 +452,33 @@ hipError_t launch_t(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) 
             default: return hipErrorNotSupported;
         }
     } else {
+        if constexpr (!DOWN && T == kQ8_0)
+            if (x32) return launch_one<T, DOWN, 8, true>(a, G, hq, hd, s);
         return launch_one<T, DOWN, 8>(a, G, hq, hd, s);
     }
 }
 
 template <bool DOWN>
-bool geom_any(int t, const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries) {
+bool geom_any(int t, const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries, bool x32) {
     MfmaGeom G;
     switch (t) {
-        case kQ4_K: return mfma_geom<kQ4_K, DOWN>(L, cap_groups, cap_entries, max_entries, G);
-        case kQ6_K: return mfma_geom<kQ6_K, DOWN>(L, cap_groups, cap_entries, max_entries, G);
-        case kQ8_0: return mfma_geom<kQ8_0, DOWN>(L, cap_groups, cap_entries, max_entries, G);
-        case kIQ4_XS: return mfma_geom<kIQ4_XS, DOWN>(L, cap_groups, cap_entries, max_entries, G);
+        case kQ4_K: return mfma_geom<kQ4_K, DOWN>(L, cap_groups, cap_entries, max_entries, false, G);
+        case kQ6_K: return mfma_geom<kQ6_K, DOWN>(L, cap_groups, cap_entries, max_entries, false, G);
+        case kQ8_0: return mfma_geom<kQ8_0, DOWN>(L, cap_groups, cap_entries, max_entries, x32 && !DOWN, G);
+        case kIQ4_XS: return mfma_geom<kIQ4_XS, DOWN>(L, cap_groups, cap_entries, max_entries, false, G);
         default: return false;
     }
 }
 
 }  // namespace
 
-bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries) {
+bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries, bool x_scale32) {
     if (mixed_gu(L) || cap_groups <= 0 || cap_entries < cap_groups) return false;
     // the DMA reads whole 16-byte chunks: a matrix's last chunk must stay inside the blob
     if (L.bytes % 16 || L.up_off % 16 || L.down_off % 16) return false;
     if (L.gu_type != kQ8_0 && canon_lanes((int)(L.n_embd / 256)) < 4) return false;
-    return geom_any<false>(L.gu_type, L, cap_groups, cap_entries, max_entries) &&
-           geom_any<true>(L.d_type, L, cap_groups, cap_entries, max_entries);
+    return geom_any<false>(L.gu_type, L, cap_groups, cap_entries, max_entries, x_scale32) &&
+           geom_any<true>(L.d_type, L, cap_groups, cap_entries, max_entries, false);
 }
 
 hipError_t launch_mfma_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) {

@@ -48,6 +48,7 @@ struct GroupedArgs {
     int max_entries;   // the most entries a group can have (the call's token count), 0 when not known
     void* hact;        // scratch: the down stream's h activations (int8 values, scales, sums of 16)
     int64_t cap_entries_hint;   // the entries the scratch was sized for
+    bool x_scale32 = false;       // the q8_1 rows may have a scale of their own in each 32-value block (a caller's rows)
 };
 hipError_t launch_native_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 hipError_t launch_native_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
@@ -59,7 +60,8 @@ hipError_t launch_stream_down(const ExpertLayout& L, const GroupedArgs& a, hipSt
 // h = SwiGLU of the gate/up scratch, per-32 q8 (int8 values, scales, sums of 16; hq's q8_1 blocks too)
 hipError_t launch_stream_h(const ExpertLayout& L, const GroupedArgs& a, int8_t* hq, float* hd, int* hs, hipStream_t s);
 // experts_mfma.hip: the same products with the units' integer sums on the matrix cores (large batches)
-bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries);
+bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries,
+                      bool x_scale32 = false);
 hipError_t launch_mfma_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 hipError_t launch_mfma_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 
