@@ -315,3 +315,51 @@ def test_iq_mmq_grouped_f16_operands(xm, t, w_rows, w_cols, counts, big):
         r0, r1 = int(bounds[e]), int(bounds[e + 1])
         want, mag = a[r0:r1] @ W[e].T, a[r0:r1].abs() @ W[e].abs().T
         assert bool(((dst[r0:r1].double() - want).abs() <= w_cols * 2.0 ** -24 * mag).all()), e
+
+
+def _iq4_with_nonfinite(xm, blk, rows, cols):
+    """IQ4_XS rows at blk whose blocks take +inf, -inf and NaN as d in turn (every fourth keeps its own; inf with some
+    sub-block scale 32 - 32 = 0, so inf x 0 too) -> the f16 operands: rounded once, saturated, NaN as -65504."""
+    b = blk.view(-1, 136)
+    for i, bits in enumerate((0x7C00, 0xFC00, 0x7E00)):
+        b[i::4, 0:2] = torch.tensor([bits & 255, bits >> 8], dtype=torch.uint8, device=DEV)
+    b[0::8, 2:4] = 0xAA          # ls = 32 + low bits in every sub-block
+    b[0::8, 4] &= 0xF0           # sub-block 0: ls = 32
+    w = xm.iq_dequant_f32(23, blk, rows * cols).reshape(rows, cols)
+    assert bool(w.isinf().any()) and bool(w.isnan().any()) and bool(w.isfinite().any())
+    return torch.where(w.isnan(), torch.full_like(w, -65504.0), w).clamp(-65504, 65504).half().double()
+
+
+def test_iq_mmq_iq4_nonfinite_scales(xm):
+    """IQ4_XS blocks whose scale is infinite or not a number: the weights saturate as everywhere in the f16 products."""
+    rows, cols, total = 256, 512, 40
+    g = torch.Generator(device=DEV).manual_seed(1)
+    blk = torch.zeros(rows * xm.row_bytes(23, cols), dtype=torch.uint8, device=DEV)
+    xm.quantize_rows(23, torch.randn(rows * cols, generator=g, device=DEV) * 0.02, out=blk)
+    W = _iq4_with_nonfinite(xm, blk, rows, cols)
+    x = torch.randn(total, cols, generator=g, device=DEV)
+    xq = xm.iq_mmq_quantize(x, None, cols, cols, total, True)
+    d = xq[total * cols:total * cols + total * (cols // 32) * 4].view(torch.float32).reshape(total, -1)
+    a = (xq[:total * cols].view(torch.int8).reshape(total, cols).float() * d.repeat_interleave(32, dim=1)).half().double()
+    ids = torch.arange(total, dtype=torch.int32, device=DEV)
+    dst = torch.zeros(total, rows, device=DEV)
+    xm.iq_mmq_grouped(23, blk, blk.numel(), rows, cols, 1, xq, total,
+                      torch.tensor([0, total], dtype=torch.int32, device=DEV), ids, dst, rows)
+    assert bool(((dst.double() - a @ W.T).abs() <= cols * 2.0 ** -24 * (a.abs() @ W.abs().T)).all())
+
+
+def test_prefill_iq4_nonfinite_scales(xm):
+    """The same in a prompt layer, whose words come by DMA: h and the output stay finite."""
+    H = F = 256
+    T = 40
+    arena, L = xm.build_arena(1, H, F, 23, 23, seed=3)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    gate, up = (_iq4_with_nonfinite(xm, arena[0, o:o + F * L.gu_row], F, H) for o in (0, L.up_off))
+    down = xm.iq_dequant_f32(23, arena[0, L.down_off:], H * F).reshape(H, F).half().double()
+    x = (torch.randn(T, H, generator=g, device=DEV) * 3e-5).half().float()
+    res, out = torch.zeros(T, H, device=DEV), torch.empty(T, H, device=DEV)
+    xm.MoeLayer(L, arena, 1, 1, T, prefill=True)(x, torch.zeros(T, 1, device=DEV), res, out)
+    h = torch.nn.functional.silu(x.double() @ gate.T) * (x.double() @ up.T)
+    assert float(h.abs().max()) < 65504
+    want = h @ down.T
+    assert float((out.double() - want).abs().max()) <= 2e-2 * float(want.abs().max())
