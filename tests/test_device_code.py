@@ -102,3 +102,22 @@ def test_the_check_sees_a_missing_wait():
     assert len(unordered_dmas(loop)[0]) == 1
     for wait in (("s_waitcnt lgkmcnt(0)", True), ("s_barrier", False)):
         assert unordered_dmas(loop[:1] + [wait] + loop[1:]) == ([], 1)
+
+
+def test_chain_accumulators_are_apart_from_their_operands(tmp_path):
+    """gemv.hip's 16-step chains write their accumulator before they have read all of their operands, so it shares no
+    register with one (an early-clobber operand: without it the compiler may share one of equal value)."""
+    sys.path.insert(0, str(CSRC.parent))
+    import build
+    asm = tmp_path / "k.s"
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", "-o", str(asm), str(CSRC / "gemv.hip")], check=True,
+                   capture_output=True)
+    runs = 0
+    for block in asm.read_text().split("#ASMSTART")[1:]:
+        regs = re.findall(r"v_fmac_f32_dpp (v\d+), (v\d+), (v\d+)", block.split("#ASMEND")[0])
+        if regs:
+            assert len(regs) == 16 and len({d for d, _, _ in regs}) == 1
+            assert all(d not in (a, b) for d, a, b in regs), regs
+            runs += 1
+    assert runs > 0
+    assert '"+&v"(acc)' in (CSRC / "gemv.hip").read_text()

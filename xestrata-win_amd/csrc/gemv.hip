@@ -184,7 +184,7 @@ __device__ __forceinline__ void chain16(float& acc, float g, const float (&b)[16
             XS_FMAC("5", "%7") XS_FMAC("6", "%8") XS_FMAC("7", "%9") XS_FMAC("8", "%10") XS_FMAC("9", "%11")
                 XS_FMAC("10", "%12") XS_FMAC("11", "%13") XS_FMAC("12", "%14") XS_FMAC("13", "%15") XS_FMAC("14", "%16")
                     XS_FMAC("15", "%17")
-        : "+v"(acc)
+        : "+&v"(acc)
         : "v"(g), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]),
           "v"(b[9]), "v"(b[10]), "v"(b[11]), "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15]));
 }
