@@ -267,3 +267,35 @@ def test_native_expert_grouped_scale_a_block(xm, xo, H, F, sizes):
     want = xo.native_expert_grouped(xo.layout(8, 8, H, F), [t2n(arena[e]) for e in experts], start, dst, tok, xq, n)
     for got in outs:
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("gu,dt,H,F,groups,T", [(12, 14, 1024, 512, 8, 1), (8, 8, 2048, 768, 4, 1), (8, 8, 2048, 768, 5, 1),
+                                                (23, 23, 2048, 768, 8, 1), (12, 12, 2048, 768, 8, 1), (12, 12, 4096, 256, 8, 3)])
+def test_grouped_of_one_entry_a_group(xm, xo, gu, dt, H, F, groups, T):
+    """As many entries as groups by capacity: on either side of the size up to which the lane-per-row kernels take them
+    (20 MiB of weights below hidden 4096), and where some groups hold several entries and others are absent all the same:
+    the oracle's bits, and a misaligned blob still sets the status word."""
+    rng = np.random.default_rng(H + groups)
+    arena, L = xm.build_arena(2, H, F, gu, dt, seed=gu + H)
+    sizes = [1] * groups if T == 1 else [T] + [1] * (groups - T)      # (fewer groups than the capacity)
+    start, tok, dst = group_case(len(sizes), sizes, T, rng)
+    n, experts = int(start[-1]), [i % 2 for i in range(len(sizes))]
+    assert n == groups
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16).float()
+    xq = xm.quantize_q8_1_rows(x.to(DEV))
+    ptrs = [arena[e].data_ptr() for e in experts]
+    d_start, d_tok, d_dst = (torch.from_numpy(v).to(DEV) for v in (start, tok, dst))
+    ng = torch.tensor([len(sizes)], dtype=torch.int32, device=DEV)
+    scratch = torch.zeros(xm.native_expert_scratch_bytes(n, F), dtype=torch.uint8, device=DEV)
+    out = torch.zeros(n, H, device=DEV)
+    print(f"[case] one entry a group {gu}/{dt} H={H} F={F} groups={groups}", flush=True)
+    xm.native_expert_grouped(L, torch.tensor(ptrs, dtype=torch.int64, device=DEV), d_start, ng, d_dst, d_tok, groups, n, xq,
+                             scratch, out)
+    want = xo.native_expert_grouped(xo.layout(gu, dt, H, F), [t2n(arena[e]) for e in experts], start, dst, tok, t2n(xq), n)
+    assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+    word = scratch[xm.native_expert_scratch_bytes(n, F) - 256:][:4].view(torch.int32)
+    assert int(word[0]) == 0
+    ptrs[0] += 8
+    xm.native_expert_grouped(L, torch.tensor(ptrs, dtype=torch.int64, device=DEV), d_start, ng, d_dst, d_tok, groups, n, xq,
+                             scratch, out)
+    assert int(word[0]) == 1

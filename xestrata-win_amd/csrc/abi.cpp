@@ -243,6 +243,23 @@ int grouped_args(const xs_expert_layout_t* L, const unsigned long long* grp_ptr,
     return ok();
 }
 
+// One entry a group and few weights: the lane-per-row kernels are ahead of the matrix-core rows, whose work-groups start
+// slower (an entry's activations beside 15 empty places, the ring, a launch for h).  known: a call of one token, for which
+// the lane-per-row kernels have an instance of one entry; else capacities of as many entries as groups (one token, or
+// few), and those kernels take four entries a pass.  Measured, lane-per-row against matrix cores, us:
+//   known: shared Q8_0 expert of hidden 1024 18.6 / 19.9, 2048 23.1 / 25.5, 4096 33.1 / 37.2, 7168 (47 MB) 45.6 / 51.6;
+//     layers of hidden 2048 Q4_K with Q8_0 down (27 MB) 31.2 / 31.8, F 1536 IQ4_XS with Q8_0 down (53 MB) 41.7 / 37.6;
+//     hidden 4096 F 768 Q4_K with Q8_0 down (55 MB) 37.8 / 39.7, Q6_K (62 MB) 60.6 / 53.2
+//   not known: hidden 1024 Q4_K/Q6_K 8 groups (8 MB) 13.4 / 14.9; 2048 IQ4_XS 8 groups (20 MB) 22.9 / 24.3, Q4_K (21 MB)
+//     26.1 / 23.2; 4096 F 768 IQ4_XS 4 groups (20 MB) 24.1 / 28.8, 8 (40 MB) 37.7 / 44.7, F 1536 Q4_K 4 (42 MB) 41.0 /
+//     43.9, Q8_0 2 (40 MB) 42.4 / 34.2, Q4_K 8 (85 MB) 85.5 / 57.6
+bool lane_rows_ahead(const xs_expert_layout_t* L, int64_t cap_groups, int64_t cap_entries, int max_entries) {
+    const bool known = max_entries == 1;
+    if (!known && (max_entries != 0 || cap_entries != cap_groups)) return false;
+    const bool wide = L->n_embd >= 4096 && (known || L->gu_type != 8);   // (8: Q8_0)
+    return cap_groups * (int64_t)L->bytes <= (wide ? 56ll << 20 : known ? 32ll << 20 : 20ll << 20);
+}
+
 // max_entries: the most entries one group can hold (the call's token count), 0 when not known.  own_rows: x_q8_1 is from
 // quantize_q8_1_rows, one scale repeated over 256 values
 int grouped_impl(const xs_expert_layout_t* L, const unsigned long long* grp_ptr, const int32_t* grp_start,
@@ -260,7 +277,8 @@ int grouped_impl(const xs_expert_layout_t* L, const unsigned long long* grp_ptr,
     const xs::ExpertLayout XL = to_layout(L);
     hipError_t e;
     // the same bits on each path
-    if (xs::mfma_rows_usable(XL, cap_groups, cap_entries, max_entries, !own_rows)) {   // the units' sums on the matrix cores
+    if (!lane_rows_ahead(L, cap_groups, cap_entries, max_entries) &&
+        xs::mfma_rows_usable(XL, cap_groups, cap_entries, max_entries, !own_rows)) {   // the units' sums on the matrix cores
         e = xs::launch_mfma_gu(XL, a, S(stream));
         if (e == hipSuccess) e = xs::launch_mfma_down(XL, a, S(stream));
     } else if (xs::stream_usable(XL, max_entries, cap_groups, cap_entries)) {   // the weight-stream kernels
