@@ -18,7 +18,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
                                                       int64_t n_embd, int k, const uint32_t* __restrict__ live) {
     const int64_t t = blockIdx.y;
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n_embd || (live && *live == 0u)) return;
+    if (c >= n_embd) return;
+    const uint32_t on = live ? *live : 1u;   // (loaded beside the parts; waited for only before the store)
     const float* p = parts + t * k * n_embd + c;
     const float* w = weights + t * k;
     float sum = p[0] * w[0];
@@ -35,7 +36,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
         sum += sv;
     }
     if (residual) sum = residual[t * n_embd + c] + sum;
-    out[t * n_embd + c] = sum;
+    if (on != 0u) out[t * n_embd + c] = sum;
 }
 
 __global__ __launch_bounds__(256) void add_inplace_kernel(float* __restrict__ x, const float* __restrict__ y, int64_t n) {
