@@ -493,3 +493,23 @@ def test_decode_batch_paths(xm, xo, T, H, F, gu, dt):
         else:
             assert layer.status() == 0
             assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("T,k", [(3, 8), (4, 6), (2, 8)])
+@pytest.mark.parametrize("gu,dt", [(23, 23), (8, 8)])
+def test_decode_wide_few_tokens(xm, xo, T, k, gu, dt):
+    """Hidden 4096, F 1536 at 2 to 4 tokens: gate/up launches on either side of one and a half rounds of work-groups (24
+    groups: 16 rows a wave; 16 groups: as many, by their own count), the oracle's bits."""
+    E, H, F = 64, 4096, 1536
+    arena, L = xm.build_arena(8, H, F, gu, dt, seed=T + gu)
+    arena = arena.repeat(E // 8, 1)
+    g = torch.Generator(device=DEV).manual_seed(T + k)
+    x = torch.randn(T, H, device=DEV, generator=g).to(torch.bfloat16).float()
+    logits, res = torch.randn(T, E, device=DEV, generator=g), torch.randn(T, H, device=DEV, generator=g)
+    layer, out = xm.MoeLayer(L, arena, E, k, T), torch.empty(T, H, device=DEV)
+    print(f"[case] wide few tokens {gu}/{dt} T={T} k={k}", flush=True)
+    layer(x, logits, res, out)
+    blobs = [t2n(arena[e]) for e in range(8)]
+    want = xo.moe_layer_decode(xo.layout(gu, dt, H, F), blobs * (E // 8), k, t2n(x), t2n(logits), t2n(res), n_threads=8)
+    assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+    assert layer.status() == 0
