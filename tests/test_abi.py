@@ -122,3 +122,16 @@ def test_mmq_grouped_refusals(xm):
     assert call(12, w=None) == E                # neither w nor wtab
     assert call(12, n=0) == xm.XS_OK
     assert call(12, tot=0) == xm.XS_OK
+
+
+def test_stream_handles(xm):
+    """One meaning of a stream however it is given: torch's default stream as an object is the explicit handle (enqueued,
+    as with no stream given), the raw handle 0 stays NULL (the call waits), and calls on host buffers wait on either."""
+    class Stream:
+        def __init__(self, h):
+            self.cuda_stream = h
+
+    assert xm._stream(Stream(0)) == xm.STREAM_LEGACY
+    assert xm._stream(Stream(64)) == 64
+    assert xm._stream(0) == 0 and xm._stream(64) == 64
+    assert xm._host_stream(Stream(0)) == 0 and xm._host_stream(0) == 0

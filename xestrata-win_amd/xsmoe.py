@@ -206,9 +206,10 @@ STREAM_LEGACY = 1
 
 def _stream(stream=None):
     """The handle of `stream` (a torch stream or a raw handle), by default torch's current stream: the call is enqueued
-    there, as torch's own operations are."""
+    there, as torch's own operations are, on the default stream too.  (The raw handle 0 is NULL: the call waits.)"""
     if stream is not None:
-        return getattr(stream, "cuda_stream", stream)
+        h = getattr(stream, "cuda_stream", None)
+        return stream if h is None else h or STREAM_LEGACY
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()) or STREAM_LEGACY
 
 
