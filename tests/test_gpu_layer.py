@@ -464,14 +464,18 @@ def test_default_stream_is_enqueued(xm, shared):
     assert torch.equal(out, want)
 
 
-@pytest.mark.parametrize("T,H,F,gu,dt", [(17, 2048, 768, 12, 14), (40, 2048, 768, 12, 14), (2, 4096, 512, 23, 23),
-                                         (12, 4096, 512, 12, 12), (24, 1024, 512, 8, 8), (16, 2048, 768, 12, 14)])
-def test_decode_batch_paths(xm, xo, T, H, F, gu, dt):
-    """The decode layer on either side of its choice of path (one persistent launch up to 16 tokens below hidden 4096,
-    24 for a small layer; else routing, matrix-core rows and combine as launches): the oracle's bits; a batch in which
-    one token's router finds fewer than k experts writes no output and sets bit 2, with or without a good call before
-    it in the same workspace, and the next good call is whole again."""
-    E, k = 16, 8 if H > 1024 else 2
+@pytest.mark.parametrize("T,E,H,F,gu,dt,chained", [
+    (16, 16, 2048, 768, 12, 14, False), (17, 16, 2048, 768, 12, 14, False), (17, 32, 2048, 768, 12, 14, True),
+    (23, 16, 2048, 768, 12, 14, False), (24, 16, 2048, 768, 12, 14, True), (40, 16, 2048, 768, 12, 14, True),
+    (23, 16, 1024, 512, 8, 8, False), (24, 16, 1024, 512, 8, 8, True), (2, 16, 4096, 512, 23, 23, True),
+    (12, 16, 4096, 512, 12, 12, True), (1, 16, 4096, 512, 12, 12, False)])
+def test_decode_batch_paths(xm, xo, T, E, H, F, gu, dt, chained):
+    """The decode layer on either side of its choice of path (one persistent launch for one token and, below hidden 4096,
+    up to 16 tokens, up to 23 while the experts within reach are under 64 MiB: 16 of this shape 47, 32 of them 93; else
+    routing, matrix-core rows and combine as launches), told by the persistent launch's call counters; the oracle's bits;
+    a batch in which one token's router finds fewer than k experts writes no output and sets bit 2, with or without a
+    good call before it in the same workspace, and the next good call is whole again."""
+    k = 8 if H > 1024 else 2
     arena, L = xm.build_arena(E, H, F, gu, dt, seed=T)
     g = torch.Generator(device=DEV).manual_seed(T + H)
     logits = torch.randn(T, E, device=DEV, generator=g)
@@ -481,7 +485,7 @@ def test_decode_batch_paths(xm, xo, T, H, F, gu, dt):
     layer = xm.MoeLayer(L, arena, E, k, T)
     bad = logits.clone()
     bad[T // 2] = float("nan")
-    print(f"[case] batch path T={T} H={H}", flush=True)
+    print(f"[case] batch path T={T} E={E} H={H}", flush=True)
     for lg in (bad, logits, bad, logits):
         out = torch.full_like(res, 7.0)
         layer(x, lg, res, out)
@@ -493,6 +497,8 @@ def test_decode_batch_paths(xm, xo, T, H, F, gu, dt):
         else:
             assert layer.status() == 0
             assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
+    counters = layer.ws[layer.ws_ptr - layer.ws.data_ptr():][128:128 + 16 * 128]   # every persistent call adds to them
+    assert bool(counters.any()) == (not chained)
 
 
 @pytest.mark.parametrize("T,k", [(3, 8), (4, 6), (2, 8)])
