@@ -217,11 +217,13 @@ def test_prefill_experts_saturation_status(xm):
         xm._check(xm.lib().xs_moe_status_check(status, None))   # clear (again)
 
 
-@pytest.mark.parametrize("T", [2, 3, 4, 5])
-@pytest.mark.parametrize("gu,H,F", [(8, 2048, 640), (8, 2048, 1408), (12, 2048, 1408), (8, 4096, 384), (8, 4096, 1536)])
+@pytest.mark.parametrize("T", [2, 3, 4, 5, 16])
+@pytest.mark.parametrize("gu,H,F", [(8, 2048, 640), (8, 2048, 1408), (12, 2048, 1408), (8, 4096, 384), (8, 4096, 1536),
+                                    (12, 1024, 384), (23, 1024, 640), (23, 4096, 384), (14, 2048, 640)])
 def test_q8_0_down_of_several_steps(xm, xo, gu, H, F, T):
     """Q8_0 down rows that the weight stream takes in several steps (F 640: 5, F 1408: 11 at up to 4 tokens), beside
-    one-step rows (F 384), more tokens, and F 1536, whose rows took two steps before the matrix-core rows: the shared
+    one-step rows (F 384), more tokens, gate/up rows of four canonical lanes (hidden 1024), Q6_K gate/up rows, which the
+    stream does not take, and F 1536, whose rows took two steps before the matrix-core rows: the shared
     expert's rows and the layer's output (hidden 4096: the stream's layers) are the oracle's bits."""
     E, k = 4, 2
     arena, L = xm.build_arena(E, H, F, gu, 8, seed=F + T)

@@ -1,6 +1,8 @@
 // xestrata-win_amd/csrc/experts_stream.hip - the grouped expert products of decode and verify windows (2-16 tokens)
 // as a weight stream: the same canonical row arithmetic as experts_decode.hip (xs_units.h, bit for bit the oracle),
-// with the memory side rebuilt for HBM bandwidth.
+// with the memory side rebuilt for HBM bandwidth.  It serves the layouts that the matrix-core rows (experts_mfma.hip) do
+// not take but whose rows have four canonical lanes or more: Q8_0 down weights with n_ff = 128 more than a multiple of
+// 256.  (One shared expert of hidden 2048, F 1408: 41 us at 2 tokens, 47 at 4, 93 at 8.)
 //
 // Work: a task is (group, R = 64 / L consecutive rows of its matrix), L the canonical lanes of a row; lane (r, c) of a
 // wave computes row r's canonical chain c over every entry of the group.  Tasks are dealt to the waves of a persistent
@@ -339,12 +341,15 @@ bool stream_geom(const ExpertLayout& L, int unit, int block_values, int block_by
 template <int T, bool DOWN, int LPR>
 hipError_t launch_lpr(const GroupedArgs& a, const StreamGeom& G, hipStream_t s, const int8_t* hq, const float* hd,
                       const int* hs) {
-    constexpr bool kWide = !DOWN && T != kQ4_K;   // the instances that fit three waves a SIMD
-    void (*kern)(GroupedArgs, StreamGeom, const int8_t*, const float*, const int*) =
-        kWide && G.waves == kStreamWavesWide
-            ? (G.ne <= 4 ? stream_kernel<T, DOWN, LPR, 4, kWide ? kStreamWavesWide : kStreamWaves>
-                         : stream_kernel<T, DOWN, LPR, 8, kWide ? kStreamWavesWide : kStreamWaves>)
-            : (G.ne <= 4 ? stream_kernel<T, DOWN, LPR, 4, kStreamWaves> : stream_kernel<T, DOWN, LPR, 8, kStreamWaves>);
+    void (*kern)(GroupedArgs, StreamGeom, const int8_t*, const float*, const int*) = nullptr;
+    if constexpr (DOWN) {
+        kern = stream_kernel<T, DOWN, LPR, 4, kStreamWaves>;
+    } else {
+        constexpr int kWide = T != kQ4_K ? kStreamWavesWide : kStreamWaves;   // the instances that fit three waves a SIMD
+        kern = G.waves == kStreamWaves
+                   ? (G.ne <= 4 ? stream_kernel<T, DOWN, LPR, 4, kStreamWaves> : stream_kernel<T, DOWN, LPR, 8, kStreamWaves>)
+                   : (G.ne <= 4 ? stream_kernel<T, DOWN, LPR, 4, kWide> : stream_kernel<T, DOWN, LPR, 8, kWide>);
+    }
     const size_t lds = (size_t)G.meta_bytes + (size_t)G.act_bytes + (size_t)G.waves * G.ring;
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -358,8 +363,7 @@ hipError_t launch_lpr(const GroupedArgs& a, const StreamGeom& G, hipStream_t s, 
 
 template <int T, bool DOWN>
 hipError_t launch_stream_t(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) {
-    constexpr int bv = T == kQ8_0 ? 32 : 256;
-    constexpr int bb = T == kQ8_0 ? 34 : T == kQ4_K ? 144 : T == kQ6_K ? 210 : 136;
+    constexpr int bv = block_values(T), bb = block_bytes(T);
     const int unit = DOWN || T == kQ8_0 ? 32 : 256;
     StreamGeom G;
     if (!stream_geom<DOWN>(L, unit, bv, bb, a.max_entries, a.cap_groups, a.cap_entries_hint, G, !DOWN && T != kQ4_K))
@@ -372,11 +376,15 @@ hipError_t launch_stream_t(const ExpertLayout& L, const GroupedArgs& a, hipStrea
         const hipError_t e = launch_stream_h(L, a, hq, hd, hs, s);
         if (e != hipSuccess) return e;
     }
-    switch (canon_lanes(G.n_in / unit)) {
-        case 8: return launch_lpr<T, DOWN, 8>(a, G, s, hq, hd, hs);
-        case 4: return launch_lpr<T, DOWN, 4>(a, G, s, hq, hd, hs);
-        default: return hipErrorNotSupported;
+    const int lanes = canon_lanes(G.n_in / unit);
+    if constexpr (DOWN) {
+        if (lanes == 4) return launch_lpr<T, DOWN, 4>(a, G, s, hq, hd, hs);
+    } else {
+        if (lanes == 8) return launch_lpr<T, DOWN, 8>(a, G, s, hq, hd, hs);
+        if constexpr (T != kQ8_0)   // (hidden sizes are whole 256s: eight Q8_0 blocks)
+            if (lanes == 4) return launch_lpr<T, DOWN, 4>(a, G, s, hq, hd, hs);
     }
+    return hipErrorNotSupported;
 }
 
 }  // namespace
@@ -385,21 +393,18 @@ bool stream_usable(const ExpertLayout& L, int n_tok, int64_t cap_groups, int64_t
     if (n_tok < 2 || n_tok > 16 || mixed_gu(L)) return false;   // (one gate/up type: the gate and up rows as one matrix)
     // the DMA reads whole 16-byte chunks: a matrix's last chunk must stay inside the blob
     if (L.bytes % 16 || L.up_off % 16 || L.down_off % 16) return false;
-    const int types[2] = {L.gu_type, L.d_type};
-    for (int t : types)
-        if (t != kQ4_K && t != kQ6_K && t != kQ8_0 && t != kIQ4_XS) return false;
+    // (the down layouts of the matrix-core rows are theirs; a step of Q6_K gate/up rows passes kStreamNiMax)
+    if (L.d_type != kQ8_0 || L.n_ff % 256 != 128) return false;
+    if (L.gu_type != kQ4_K && L.gu_type != kQ8_0 && L.gu_type != kIQ4_XS) return false;
     StreamGeom G;
-    const int gbv = L.gu_type == kQ8_0 ? 32 : 256, dbv = L.d_type == kQ8_0 ? 32 : 256;
-    auto bytes = [](int t) { return t == kQ8_0 ? 34 : t == kQ4_K ? 144 : t == kQ6_K ? 210 : 136; };
-    return stream_geom<false>(L, L.gu_type == kQ8_0 ? 32 : 256, gbv, bytes(L.gu_type), n_tok, cap_groups, cap_entries,
-                              G) &&
-           stream_geom<true>(L, 32, dbv, bytes(L.d_type), n_tok, cap_groups, cap_entries, G);
+    const bool q8 = L.gu_type == kQ8_0;
+    return stream_geom<false>(L, q8 ? 32 : 256, q8 ? 32 : 256, block_bytes(L.gu_type), n_tok, cap_groups, cap_entries, G) &&
+           stream_geom<true>(L, 32, 32, block_bytes(kQ8_0), n_tok, cap_groups, cap_entries, G);
 }
 
 hipError_t launch_stream_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) {
     switch (L.gu_type) {
         case kQ4_K: return launch_stream_t<kQ4_K, false>(L, a, s);
-        case kQ6_K: return launch_stream_t<kQ6_K, false>(L, a, s);
         case kQ8_0: return launch_stream_t<kQ8_0, false>(L, a, s);
         case kIQ4_XS: return launch_stream_t<kIQ4_XS, false>(L, a, s);
         default: return hipErrorNotSupported;
@@ -407,13 +412,7 @@ hipError_t launch_stream_gu(const ExpertLayout& L, const GroupedArgs& a, hipStre
 }
 
 hipError_t launch_stream_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s) {
-    switch (L.d_type) {
-        case kQ4_K: return launch_stream_t<kQ4_K, true>(L, a, s);
-        case kQ6_K: return launch_stream_t<kQ6_K, true>(L, a, s);
-        case kQ8_0: return launch_stream_t<kQ8_0, true>(L, a, s);
-        case kIQ4_XS: return launch_stream_t<kIQ4_XS, true>(L, a, s);
-        default: return hipErrorNotSupported;
-    }
+    return L.d_type == kQ8_0 ? launch_stream_t<kQ8_0, true>(L, a, s) : hipErrorNotSupported;
 }
 
 }  // namespace xs
