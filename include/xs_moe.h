@@ -68,7 +68,8 @@ int xs_quantize_q8_1_rows(const float* x, int64_t n_rows, int64_t n_cols, void* 
 
 /* Grouped experts in the native format (decode and verify windows).  Group g's blob is at device address
  * grp_ptr[g]; its entries [grp_start[g], grp_start[g+1]) read token ent_tok[e]'s q8_1 row (n_embd/32 blocks a token
- * in x_q8_1) and write row ent_dst[e] of `out` (n_embd floats).  Counts are read on the device; grid_groups (0:
+ * in x_q8_1; Q8_0 gate/up rows take each 32-value block's own scale, the other types the scale of the first of each 8)
+ * and write row ent_dst[e] of `out` (n_embd floats).  Counts are read on the device; grid_groups (0:
  * cap_groups) rows of work-groups stride over the groups.  Replaces native_expert_grouped
  * (include/strata/kernels/iq_kernels.hpp:90-93; src/kernels/xe/iq_kernels.cpp:2042-2178).  A NULL stream runs on
  * the default stream and synchronises.  A blob address that is not 16-byte aligned is skipped and flagged in the
@@ -251,16 +252,19 @@ int xs_add_inplace(float* x, const float* y, int64_t n, void* stream);
  * arena + e * blob_bytes): router -> plan -> q8_1 -> grouped experts -> combine -> residual.
  * out = residual + MoE(x); out may equal residual.  workspace: xs_moe_layer_decode_workspace_bytes for the largest
  * n_tok it will serve, 256-byte aligned, zeroed once before its first call (every call leaves it ready for the next).
- * The layer runs as one persistent launch for one token and, below hidden 4096, up to 16 tokens (24 for small layers) of
- * the formats Q4_K/Q6_K, Q4_K/Q4_K, Q8_0/Q8_0, IQ4_XS/IQ4_XS (n_tok * k <= 256); else as the chain of kernels below.  The engine's moe_route + moe_finish
- * surface (include/strata/core/layer.hpp:108-199) on one GPU, without the host ring. */
+ * The layer runs as one persistent launch where its formats are Q4_K/Q6_K, Q4_K/Q4_K, Q8_0/Q8_0 or IQ4_XS/IQ4_XS, n_tok <= 64
+ * and n_tok * k <= 256, for one token and, below hidden 4096, for up to 16 tokens, up to 23 while min(n_tok * k, n_expert)
+ * blobs are under 64 MiB; at more tokens too where the matrix-core rows do not take the layout (K-quant or IQ4_XS gate/up
+ * rows of a hidden size that is no multiple of 1024; Q8_0 down rows of n_ff no multiple of 256, at hidden 4096 and more only
+ * past 16 tokens or where the weight stream does not take them either).  Else as the chain of kernels below.  The engine's
+ * moe_route + moe_finish surface (include/strata/core/layer.hpp:108-199) on one GPU, without the host ring. */
 int xs_moe_layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_bytes, int n_expert, int k,
                         const float* x, const float* logits, const float* residual, float* out, int n_tok,
                         void* workspace, size_t workspace_bytes, void* stream);
 size_t xs_moe_layer_decode_workspace_bytes(const xs_expert_layout_t* L, int n_expert, int k, int n_tok);
 /* Device address of the decode workspace's status word: 0 after good calls; bit 1 a wait of the persistent layer
- * passed its bound (50 ms), bit 2 a token's router produced fewer than k experts (NaN logits) - that call wrote no
- * output.  Bits stay set until the caller clears the word; the workspace itself needs no reset after an error.  No
+ * passed its bound (50 ms), bit 2 a token's softmax router produced fewer than k experts (NaN logits) - that call wrote
+ * no output (the grouped sigmoid router gives such a token ids in range and NaN weights).  Bits stay set until the caller clears the word; the workspace itself needs no reset after an error.  No
  * counterpart in the reference (its layer reports through host-side checks of each launch). */
 int32_t* xs_moe_layer_decode_status(void* workspace);
 /* The checked contract of the persistent layer: synchronises `stream`, reads the status word; 0 -> XS_OK; else clears

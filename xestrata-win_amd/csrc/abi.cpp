@@ -966,10 +966,10 @@ int layer_decode(const xs_expert_layout_t* L, const uint8_t* arena, size_t blob_
     xs::FusedPlan P;
     // The chained path (routing, gate/up, h, down, combine) on the matrix-core rows or the weight stream, measured faster
     // than the persistent layer from 2 tokens of a wide layer on (hidden >= 4096; hidden 4096 IQ4_XS at 8 and 16 tokens
-    // 219 and 394 us against 565 and 502, hidden 7168 Q4_K at 6: 353 against 762) and for more than 16 tokens of a
+    // 195 and 329 us against 565 and 502, hidden 7168 Q4_K at 6: 353 against 762) and for more than 16 tokens of a
     // narrower one (hidden 2048, Q4_K/Q6_K: 17 tokens 135 against 154 us, 24 133 against 195, 32 140 against 239; the
     // persistent layer stays ahead up to 16: 124 against ~130).  A layer of few, small experts (8 of 1.7 MB, hidden 1024)
-    // is bound by the chain's launches up to ~24 tokens: 20 tokens 39 against 33 us, 24 32 against 39.
+    // is bound by the chain's launches below 24 tokens: 20 tokens 39 against 33 us, 24 32 against 39.
     const int64_t groups = capx < n_expert ? capx : n_expert;
     const bool rows = xs::mfma_rows_usable(XL, groups, capx, n_tok);
     const bool chained = L->n_embd >= 4096 ? n_tok >= 2 && (rows || xs::stream_usable(XL, n_tok, groups, capx))

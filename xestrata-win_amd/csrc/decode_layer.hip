@@ -1,7 +1,8 @@
 // xestrata-win_amd/csrc/decode_layer.hip - the decode layer's routing in one launch: the tokens' q8_1 activations,
-// the softmax top-k of every token and the plan over their routed entries.  Work-group 0 (16 waves) routes and plans;
-// work-groups 1.. quantize the activations beside it, 1024-lane rounds each (in work-group 0 after its routing they
-// took more than half the launch: 10.7 of 20 us at 8 tokens of hidden 4096).  The
+// the softmax top-k of every token and, up to 16 tokens, the plan over their routed entries: work-group 0 (16 waves)
+// routes and plans then; more tokens take a work-group for each 16, and the plan a launch of its own.  The work-groups past
+// those quantize the activations beside them, 1024-lane rounds each (in work-group 0 after its routing they took more than
+// half the launch: 10.7 of 20 us at 8 tokens of hidden 4096).  The
 // reference runs these as quantize_q8_1_rows, router_top10 and resident_plan (src/core/verify.cpp:1160-1360, the
 // resident verify window) or routes on the device and plans on the host (src/core/moe_window.cpp:183-250); one launch
 // here instead of three, on the same arithmetic (xs_route.h).

@@ -1,4 +1,6 @@
-// xestrata-win_amd/csrc/experts_decode.hip - grouped expert products for decode and verify windows (1-16 tokens):
+// xestrata-win_amd/csrc/experts_decode.hip - grouped expert products for decode and verify windows (1-16 tokens), in use
+// for one entry a group and few weights (the rule's figures are beside it in abi.cpp), for mixed gate/up rows, and for the
+// layouts that the matrix-core rows and the weight stream do not take:
 // the MI355X form of the reference's native_expert_grouped (src/kernels/xe/iq_kernels.cpp:2042-2178; gate/up rows
 // :997-1031, the SwiGLU + q8_1 pass :2118-2133, down rows :1033-1063).
 //

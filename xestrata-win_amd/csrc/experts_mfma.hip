@@ -18,8 +18,9 @@
 // instructions an entry for each 32 values and lane; above ~2 entries a group that work, not the weights, bounded them.
 // Bound here by the weight stream and each work-group's start (indices, activations, the first slice: ~5 us).  Measured,
 // 512 entries of 128 experts, hidden 2048, F 768, Q4_K: gate/up 65 us (3.5 TB/s) and down 54 (2.1) against 219 and 231;
-// layers, before and after: 64 tokens of that shape with a gated shared expert 885 -> 166 us, hidden 4096 IQ4_XS at 8
-// tokens 254 -> 195 and at 24 663 -> 431, Q4_K/Q6_K at 8 331 -> 219, hidden 7168 Q4_K at 6 tokens 762 -> 353.
+// layers, before and after: 64 tokens of that shape with a gated shared expert 885 -> 167 us, hidden 4096 IQ4_XS at 8
+// tokens 254 -> 195 and at 24 663 -> 431, Q4_K/Q6_K at 8 331 -> 192, hidden 7168 Q4_K at 6 tokens 762 -> 353.  One entry a
+// group and few weights: the lane-per-row kernels stay ahead (lane_rows_ahead, abi.cpp).
 #include "xs_device.h"
 #include "xs_kernels.h"
 #include "xs_units.h"

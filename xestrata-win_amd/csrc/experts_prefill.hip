@@ -351,7 +351,7 @@ __device__ __forceinline__ f16x8_t q8_frag(const uint4& Q, int kk, uint32_t dbit
 // them; level and scale are multiplied in fp32, where the product is exact ((level + 128) dl - 128 dl: 25 and 24 bits,
 // one fma), and rounded to f16 once, saturating (the kernel sets MODE's FP16_OVFL).  Bound by these ~18 VALU
 // instructions a four codes beside the weight stream; reading each code's byte and level on its own took 5 times as
-// long (hidden 4096, F 1536, 333 tokens: the layer 3,190 -> 656 us; gate/up 2,240, down 944 before).
+// long (hidden 4096, F 1536, 333 tokens: the layer 3,190 -> 656 us, 522 with the words by DMA; gate/up 2,240, down 944 before).
 struct Iq4Table {
     uint32_t t[4];
 };
@@ -366,7 +366,7 @@ __device__ __forceinline__ Iq4Table make_iq4_table() {   // kvalues_iq4nl + 128,
 // A block's d for its sub-blocks' scales, and what is added to their biases.  With an infinite d each value saturates by
 // its sign, and inf x 0 and a NaN d give -65504, as sat_f16x2 has them: d held to +-2^21 (a level times a scale is then 0 or
 // past the f16 range; 0 for a NaN) beside an offset of -2^17.  Once a block (hidden 4096, 333
-// tokens: the layer 0.9% slower; done to every sub-block's scale and bias 1.4%, behind a branch on the wave's rows 2.2%).
+// tokens: 519.7 -> 521.7 us a layer; done to every sub-block's scale and bias 1.4%, behind a branch on the wave's rows 2.2%).
 struct Iq4Head {
     float d, low;
 };

@@ -16,9 +16,8 @@
 //     memory tree s[t] += s[t + off], off = tpr / 2 ... 1.
 //
 // MI355X layout: a 32-lane group is half a wave64 (a xor below 32 stays inside it), so the warp form takes two rows a
-// wave and the mmvf form's 32-thread groups are wave halves.  The gemm_rows form tiles 64 tokens x 64 rows a
-// work-group, K through LDS 32 at a time stored K-major so a thread's 4 tokens and 4 rows are one 16-byte LDS read
-// each; its 16 chains stay in registers.
+// wave and the mmvf form's 32-thread groups are wave halves.  The gemm_rows form gives a work-group 16 or 64 rows of one
+// side over its lanes (staged through LDS) x 16 of the other (a value a lane, broadcast by the multiply-add itself).
 #include "xs_device.h"
 #include "xs_kernels.h"
 
@@ -166,8 +165,9 @@ template hipError_t launch_mmvf<uint16_t>(const float*, int64_t, const uint16_t*
 //     kk broadcast block kk.  A row is then read by fewer work-groups (8 group rows a wave in two accumulators, two
 //     waves a work-group: 2048 tokens 34.6 us against 26.3).
 // Chains are 1024 to 7168 steps long and few (2048 tokens x 128 experts: 4 a lane of the whole chip), so their length
-// is what bounds a router: about 14 cycles a step as measured.  The loads ahead must not stop it: two steps ahead through
-// registers, then LDS.  A tile of 64 x 64 chains a work-group, 4 x 4 a thread, read from LDS a k at a time and waiting
+// is what bounds a router: 12 ns a step as measured (25 us for 2048 steps), about 29 cycles at 2.4 GHz, in which a wave
+// reads 16 bytes a lane for each 4 steps from LDS, then runs 16 dependent products.  The loads ahead must not stop it: two
+// steps ahead through registers, then LDS.  A tile of 64 x 64 chains a work-group, 4 x 4 a thread, read from LDS a k at a time and waiting
 // for each step's loads, took 230 us at 2048 tokens x 128 experts x 2048 (now 25; 62 against 17 TFLOP/s at 4096 x 256 x
 // 7168), and 165 us for one weight row x 64 tokens x 2048 (now 13).
 struct __attribute__((packed, aligned(4))) F4u {   // 16 bytes at any float's address

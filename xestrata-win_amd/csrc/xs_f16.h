@@ -14,7 +14,7 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 __host__ __device__ constexpr int perm8(int i) { return (i == 1 || i == 5) ? i + 1 : (i == 2 || i == 6) ? i - 1 : i; }
 __host__ __device__ constexpr int perm64(int p) { return 8 * perm8(p >> 3) + perm8(p & 7); }
 
-__device__ __forceinline__ uint32_t sat_f16x2(float a, float b) {   // RNE, saturated to the f16 range (NaN kept)
+__device__ __forceinline__ uint32_t sat_f16x2(float a, float b) {   // RNE, saturated to the f16 range (NaN: -65504)
     a = __builtin_fminf(__builtin_fmaxf(a, -65504.0f), 65504.0f);
     b = __builtin_fminf(__builtin_fmaxf(b, -65504.0f), 65504.0f);
     return __builtin_bit_cast(uint32_t, (h2_t){(_Float16)a, (_Float16)b});

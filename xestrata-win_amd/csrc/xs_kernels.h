@@ -52,14 +52,14 @@ struct GroupedArgs {
 };
 hipError_t launch_native_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 hipError_t launch_native_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
-// experts_stream.hip: the same products as a weight stream (2..16 tokens, the four formats)
+// experts_stream.hip: the same products as a weight stream (2..16 tokens; Q8_0 down rows of n_ff % 256 == 128)
 bool stream_usable(const ExpertLayout& L, int n_tok, int64_t cap_groups, int64_t cap_entries);
 hipError_t launch_stream_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 hipError_t launch_stream_down(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
 
 // h = SwiGLU of the gate/up scratch, per-32 q8 (int8 values, scales, sums of 16; hq's q8_1 blocks too)
 hipError_t launch_stream_h(const ExpertLayout& L, const GroupedArgs& a, int8_t* hq, float* hd, int* hs, hipStream_t s);
-// experts_mfma.hip: the same products with the units' integer sums on the matrix cores (large batches)
+// experts_mfma.hip: the same products with the units' integer sums on the matrix cores
 bool mfma_rows_usable(const ExpertLayout& L, int64_t cap_groups, int64_t cap_entries, int64_t max_entries,
                       bool x_scale32 = false);
 hipError_t launch_mfma_gu(const ExpertLayout& L, const GroupedArgs& a, hipStream_t s);
