@@ -519,3 +519,36 @@ def test_decode_wide_few_tokens(xm, xo, T, k, gu, dt):
     want = xo.moe_layer_decode(xo.layout(gu, dt, H, F), blobs * (E // 8), k, t2n(x), t2n(logits), t2n(res), n_threads=8)
     assert np.array_equal(t2n(out).view(np.uint32), want.view(np.uint32))
     assert layer.status() == 0
+
+
+def test_decode_batch_graph_replays(xm, c2_arena, c2_shared):
+    """The chained decode layer (64 tokens, a gated shared expert) captured in a HIP graph: replays with other routings and
+    activations in the captured buffers, and eager work and waits between them, give the eager call's bits."""
+    arena, L = c2_arena
+    sh_arena, SL, w_gate = c2_shared
+    T = 64
+    g = torch.Generator(device=DEV).manual_seed(81)
+    draw = lambda *shape: torch.randn(*shape, device=DEV, generator=g)   # noqa: E731
+    x, logits, res, out = draw(T, L.n_embd), draw(T, 128), draw(T, L.n_embd), torch.zeros(T, L.n_embd, device=DEV)
+    layer, other = (xm.MoeLayer(L, arena, 128, 8, T, shared=(SL, sh_arena[0], w_gate)) for _ in range(2))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    print("[case] chained decode, graph replays", flush=True)
+    with torch.cuda.stream(s):
+        layer(x, logits, res, out, stream=s)   # warm-up on the capture stream
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            layer(x, logits, res, out, stream=s)
+    torch.cuda.synchronize()
+    for r in range(4):
+        x.copy_(draw(T, L.n_embd))
+        logits.copy_(draw(T, 128) * (1 + r))   # (ever fewer distinct experts)
+        out.zero_()
+        eager = torch.empty_like(res)
+        other(x, logits, res, eager)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int32), eager.view(torch.int32)), r
+    assert layer.status() == 0
